@@ -867,9 +867,9 @@ FusedSplit fused_split(const Grid& g, int L) {
 
 // Work split of the pair step (two steps per launch): tiles of 60 x 13
 // owned cells whose lanes cover x = 60 t - 2 .. 60 t + 61; x-interior tiles
-// have all of them in [M, nx - M - 1].  z chunks of 48 planes (32: 3.35 ms,
-// 64: 3.32 ms against 3.29 ms per launch at 1024x512x256; BZH_PAIR_KZ
-// overrides it); each chunk recomputes two planes of the first step.
+// have all of them in [M, nx - M - 1].  z chunks of pair_kz planes
+// (BZH_PAIR_KZ overrides it); each chunk recomputes two planes of the first
+// step.
 //
 // The x-interior tiles whose 16 rows all lie clear of the y faces and y CPML
 // slabs, over the z range whose chunks' iterations all lie clear of the z
@@ -891,10 +891,34 @@ struct PairSplit {
   bool has_core = false;
 };
 
-int pair_kz() {
-  int kz = 48;
-  if (const char* env = std::getenv("BZH_PAIR_KZ")) kz = std::max(1, std::atoi(env));
-  return kz;
+// Chunk depth of a pair launch.  A block marches kz owned planes plus three to
+// four of start-up and lag, one 16-wave block per CU, so a launch of B blocks
+// takes about max(B, 256) (kz + 3): below 256 blocks shorter chunks are free
+// parallelism, above it they only add start-up planes.  The chunk count that
+// minimizes this, with chunks of 3 to 48 planes (2-plane chunks measured 25 %
+// slower than 3 at 40x60x80), per step with a plane source and a flux plane:
+// 64x96x128 153 -> 49 us, 97x150x263 179 -> 111 us, 40x60x80 147 -> 35 us,
+// 128x256x512 253 -> 249 us, against 48 planes at every size.
+// ``fixed``: stochastic bfloat16 rounding draws by block, so its schedule
+// (and with it every rounded bit) stays that of 48-plane chunks.
+constexpr int kPairBlocks = 256;
+constexpr int kPairKzMin = 3, kPairKzMax = 48;
+int pair_kz(int64_t tiles, int planes, bool fixed) {
+  if (const char* env = std::getenv("BZH_PAIR_KZ")) return std::max(1, std::atoi(env));
+  if (fixed || tiles <= 0) return kPairKzMax;
+  int best = 0;
+  int64_t best_cost = 0;
+  for (int n = (planes + kPairKzMax - 1) / kPairKzMax; n <= planes; ++n) {
+    const int kz = (planes + n - 1) / n;
+    if (best > 0 && kz < kPairKzMin) break;
+    const int64_t blocks = tiles * ((planes + kz - 1) / kz);
+    const int64_t cost = std::max<int64_t>(blocks, kPairBlocks) * (kz + 3);
+    if (best == 0 || cost < best_cost) {
+      best = kz;
+      best_cost = cost;
+    }
+  }
+  return best;
 }
 
 // Finish a box: z chunking over [z0, zsplit) and [zhi, z1) with chunks of at
@@ -918,14 +942,14 @@ bool finish_box(PairBox& b, int kz, bool even) {
   return true;
 }
 
-PairSplit pair_split(const Grid& g, int L) {
+PairSplit pair_split(const Grid& g, int L, bool fixed_kz) {
   const int W = kPairCols, TY = kPairRows;
   const int Tx = (g.nx + 1 + W - 1) / W, Ty = (g.ny + 1 + TY - 1) / TY, planes = g.nz + 1;
   const int M = std::max(L, 1);
   int tx0 = (M + 2 + W - 1) / W;                           // W tx0 - 2 >= M
   int tx1 = g.nx - M - 2 >= 0 ? std::min((g.nx - M - 2) / W, Tx) : 0;  // W tx1 <= nx - M - 2
   if (tx1 <= tx0) tx0 = tx1 = 0;
-  const int kz = pair_kz();
+  const int kz = pair_kz(int64_t{Tx} * Ty, planes, fixed_kz);
   // core rows: 13 by - 2 >= M and 13 by + 13 <= ny - L - 1
   const int cy0 = (M + 2 + TY - 1) / TY;
   const int cy1 = g.ny - L - 1 - TY >= 0 ? (g.ny - L - 1 - TY) / TY + 1 : 0;
@@ -1632,7 +1656,7 @@ bool run_program(hipStream_t s, ProgramIn& in) {
         pp.mbox_n = mon_m;
       }
       // the shell launch (general kernel), then the core launch
-      const PairSplit sp = pair_split(g, pp.f.L);
+      const PairSplit sp = pair_split(g, pp.f.L, pp.f.bf16_sr != 0);
       pp.nbox = sp.nshell;
       for (int b = 0; b < sp.nshell; ++b) pp.box[b] = sp.shell[b];
       pp.core = 0;
