@@ -27,7 +27,7 @@ forward runs (``optimization/topology.py:314-342``).
 
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 
 import numpy as np
 import torch
@@ -141,7 +141,8 @@ class AdjointProblem2D:
         while done < self.steps:
             n = min(self.checkpoint, self.steps - done)
             if keep:
-                checkpoints.append(_clone_state(state))
+                # (without the workspace, whose contents do not outlive a call)
+                checkpoints.append(_clone_state(state._replace(fields_b=())))
             state = runtime.advance(state, prog, n)
             done += n
         torch.cuda.synchronize()
@@ -211,29 +212,23 @@ class AdjointProblem2D:
         adj.grad = native.buffer(grad)
 
         state = _clone_state(fwd.checkpoints[0])
-        # The recompute steps one state one step at a time: its program call
-        # and the record call are described once (the segments restore the
-        # checkpoints into the same tensors).  Building the program call anew
-        # took ~170 us of host time per step, several times the step's
-        # kernels on a 600 x 600 grid.
-        step = runtime.prepare_chunk(state, prog, 1)
-        rec = native.PreparedAdjointRecord(adj, state.hx, state.hy) if step is not None else None
+        # A segment is recomputed in one call that records every step's curl
+        # (the monitors' DFT is not part of it); the segments restore the
+        # checkpoints into the same tensors, so the call is marshalled once.
+        bare = replace(prog, monitors=[], packed_monitors=(), monitor_boxes=None)
+        step = runtime.prepare_chunk(state, bare, 1)
         nseg = len(fwd.checkpoints)
         for seg in range(nseg - 1, -1, -1):
             first = seg * K
             count = min(K, self.steps - first)
             _copy_state(state, fwd.checkpoints[seg])
-            for k in range(count):
-                # one forward step of the segment, then record the curl of H'
-                if step is not None:
-                    step()
-                else:
+            if step is not None:
+                step.recompute(adj, count, 0)
+            else:
+                for k in range(count):
                     state = runtime.run_chunk(state, prog, 1)
-                state.current_step.fill_(first + k + 1)
-                state.t.fill_(prog.t0 + (first + k + 1) * prog.dt)
-                if rec is not None:
-                    rec(k)
-                else:
+                    state.current_step.fill_(first + k + 1)
+                    state.t.fill_(prog.t0 + (first + k + 1) * prog.dt)
                     native.call_adjoint_record(adj, state.hx, state.hy, k)
             native.call_adjoint_reverse(adj, first + count - 1, count, count - 1,
                                         abi.FLAG_GRAPH_CACHE)

@@ -344,7 +344,8 @@ void run_phase(hipStream_t s, const PhaseParams& p, int phase, const Grid& g) {
 
 // ---- schedule ------------------------------------------------------------------
 enum class Kind : int32_t {
-  kPhase3d, kPhaseTm, kSource, kDft, kFused, kBatch2d, kAdjoint, kPair, kMonBox
+  kPhase3d, kPhaseTm, kSource, kDft, kFused, kBatch2d, kAdjoint, kPair, kMonBox, kTm, kDftCapture,
+  kAdjointRecord
 };
 
 struct Launch {
@@ -414,6 +415,24 @@ void enqueue(hipStream_t s, const Launch& l) {
       PairParams p;
       std::memcpy(&p, l.bytes.data(), sizeof(p));
       launch_pair3d(s, p, l.dtype);
+      break;
+    }
+    case Kind::kTm: {
+      TmParams p;
+      std::memcpy(&p, l.bytes.data(), sizeof(p));
+      launch_tm(s, p);
+      break;
+    }
+    case Kind::kDftCapture: {
+      DftCapParams p;
+      std::memcpy(&p, l.bytes.data(), sizeof(p));
+      launch_dft_capture(s, p);
+      break;
+    }
+    case Kind::kAdjointRecord: {
+      AdjointRecordParams p;
+      std::memcpy(&p, l.bytes.data(), sizeof(p));
+      launch_adjoint_record(s, p.p, p.hx, p.hy);
       break;
     }
     case Kind::kMonBox: {
@@ -756,6 +775,12 @@ struct ProgramIn {
   // reference): host s32[M, 6, 6] boxes of the cells each monitor component
   // gathers, which lets pair launches capture them densely
   const bzh_buffer* mon_boxes;
+  // optional last argument of the in-place layouts (no counterpart in the
+  // reference): f32 device workspace that lets 2D programs run several steps
+  // per launch
+  const bzh_buffer* workspace;
+  // adjoint recompute: record the forward curl of step k in slot slot + k
+  const Adjoint2dParams* record;
 };
 
 // Work split of the fused step -- the counterpart of the reference's
@@ -1354,6 +1379,208 @@ bool metrics_empty(const PhaseIn& ph) {
   return true;
 }
 
+// ---- 2D programs, several steps per launch (tm_steps.hip) -----------------------
+// Steps per launch and rows per lane (blocks of 64 columns by 32 rows).  More
+// steps spread a launch's fixed cost (about 8 us of start-up chain) and its
+// halo's reads over more of them but shrink the owned part; with fewer than
+// one block per CU the launch lasts as long as its slowest block, which 16
+// waves of two rows finish sooner than 8 of four.  us per launch step, two
+// flux lines and a line source: 200x400 (117 tiles of 48 x 16) 15.0 / 8 with
+// two rows and 18.4 / 8 with four, 1201x1603 (2584 tiles) 77.7 / 8 and
+// 55.4 / 8, there 39.2 / 6 and 28.8 / 4 with four rows; 450x450 (290 tiles)
+// measured equal, 600x600 (494) 8 % faster with four rows.  BZH_TM_T overrides
+// the steps.
+struct TmShape {
+  int T, rpt;
+};
+TmShape tm_shape(int ny, int nx) {
+  const int64_t tiles = int64_t{(nx + 48) / 48} * ((ny + 16) / 16);
+  TmShape t{tiles <= 2048 ? 8 : 6, tiles <= 256 ? 2 : 4};
+  if (const char* env = std::getenv("BZH_TM_T")) t.T = std::max(2, std::min(std::atoi(env), kTmMaxSteps));
+  return t;
+}
+
+// The source slabs of group gi (E components of ``timing`` 0 or 2, H of 1).
+bool add_tm_slabs(TmSim& d, const SourceGroupIn& grp, int comp, const bzh_buffer& field,
+                  bool post, int metallic) {
+  const int n = group_slabs(grp);
+  if (n == 0) return true;
+  const bzh_buffer& c = *grp.coeffs;
+  BZH_REQUIRE(c.element_type == BZH_F32 && grp.waves->element_type == BZH_F32 &&
+                  grp.starts->element_type == BZH_S32,
+              "source groups are f32 coefficients, f32 waveforms and s32 starts");
+  BZH_REQUIRE(grp.waves->rank == 2 && grp.waves->dims[0] == n && grp.waves->dims[1] >= 1,
+              "source waveforms must be [n, T]");
+  BZH_REQUIRE(grp.starts->rank == 2 && grp.starts->dims[0] == n && grp.starts->dims[1] == 3,
+              "source starts must be s32[n, 3]");
+  BZH_REQUIRE(c.rank == 4, "source coefficients must be [n, sz, sy, sx]");
+  if (d.nslab + n > kMaxTmSlabs) return false;
+  int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+  if (post) mask_ends(comp, metallic, false, lo, hi);
+  const int64_t cells = c.dims[1] * c.dims[2] * c.dims[3];
+  for (int i = 0; i < n; ++i) {
+    TmSlab& q = d.slab[d.nslab++];
+    q.coeff = static_cast<const float*>(c.data) + i * cells;
+    q.T = static_cast<int>(grp.waves->dims[1]);
+    q.wave = static_cast<const float*>(grp.waves->data) + static_cast<int64_t>(i) * q.T;
+    q.start = static_cast<const int32_t*>(grp.starts->data) + 3 * i;
+    q.sz = static_cast<int>(c.dims[1]);
+    q.sy = static_cast<int>(c.dims[2]);
+    q.sx = static_cast<int>(c.dims[3]);
+    q.comp = comp == kEz ? 2 : comp - kHx;
+    q.fy = static_cast<int>(field.dims[0]);
+    q.fx = static_cast<int>(field.dims[1]);
+    q.mb = lo[1];
+    q.mt = hi[1];
+    q.ml = lo[2];
+    q.mr = hi[2];
+  }
+  return true;
+}
+
+// Can a 2D program run several steps per launch?  Fills the launch's
+// parameters (bank A and the workspace bank, sources, captured boxes) and the
+// captured DFT.  float32 fields and CPML memories, scalar H coefficients, one
+// CPML thickness (or none), isotropic spacing, up to kMaxTmSlabs slabs and
+// kMaxMonBoxes monitors with host boxes, and a workspace that holds bank B
+// and the capture; everything else runs the per-phase schedule, with bitwise
+// the same results.
+bool tm_program(const ProgramIn& in, const Grid& g, TmParams& p, DftCapParams& dc, int slots) {
+  if (g.is3d || g.dtype != BZH_F32 || in.bank_b[0] != nullptr || in.nsteps < 2 || in.noalloc ||
+      in.workspace == nullptr || !metrics_empty(in.h) || !metrics_empty(in.e))
+    return false;
+  const bool cpml = in.h.nterms > 0 || in.e.nterms > 0;
+  if (cpml && (in.uniform_l <= 0 || in.h.nterms != 2 || in.e.nterms != 2)) return false;
+  for (int q : {0, 1, 3, 4})
+    if (in.h.mat[q] == nullptr || numel(*in.h.mat[q]) != 1) return false;
+  const bzh_buffer &ez = *in.bank_a[kEz], &hx = *in.bank_a[kHx], &hy = *in.bank_a[kHy];
+  if (coef_ids(in.e, 2, numel(ez))) return false;
+  std::memset(&p, 0, sizeof(p));
+  std::memset(&dc, 0, sizeof(dc));
+  PhaseIn h = in.h, e = in.e;
+  for (int c = 0; c < 3; ++c) {
+    h.tin[c] = h.tout[c] = e.src[c] = in.bank_a[kHx + c];
+    e.tin[c] = e.tout[c] = h.src[c] = in.bank_a[kEx + c];
+  }
+  const PhaseParams hp = make_phase(h, BZH_PHASE_H, g, in.dt, in.resolution, in.metallic, in.uniform_l);
+  const PhaseParams ep = make_phase(e, BZH_PHASE_E, g, in.dt, in.resolution, in.metallic, in.uniform_l);
+  if (ep.scf_f16) return false;
+  TmSim& d = p.sim;
+  d.ny = g.ny;
+  d.nx = g.nx;
+  d.metallic = in.metallic;
+  d.inv_dx = hp.inv_dx;
+  d.e_dec = ep.dec[2];
+  d.e_src = ep.scf[2];
+  d.dec_st = ep.dec_st[2];
+  d.src_st = ep.scf_st[2];
+  for (int c = 0; c < 2; ++c) {
+    d.h_dec[c] = hp.dec[c];
+    d.h_src[c] = hp.scf[c];
+  }
+  float* ws = static_cast<float*>(in.workspace->data);
+  const size_t have = ws ? static_cast<size_t>(numel(*in.workspace)) : 0;
+  size_t used = 0;
+  auto take = [&](int64_t n) {
+    float* at = ws + used;
+    used += (static_cast<size_t>(n) + 63) / 64 * 64;
+    return at;
+  };
+  d.ez[0] = static_cast<float*>(ez.data);
+  d.hx[0] = static_cast<float*>(hx.data);
+  d.hy[0] = static_cast<float*>(hy.data);
+  d.ez[1] = take(numel(ez));
+  d.hx[1] = take(numel(hx));
+  d.hy[1] = take(numel(hy));
+  if (cpml) {
+    d.L = in.uniform_l;
+    for (int t = 0; t < 4; ++t) {
+      const DevTerm& tm = t < 2 ? hp.term[t] : ep.term[t - 2];
+      if (tm.psi == nullptr || tm.psi_bf16 || tm.low != 2 * d.L || 2 * d.L > tm.n) return false;
+      d.ta[t] = tm.a;
+      d.tb[t] = tm.b;
+      d.tk[t] = tm.ik;
+      d.psi[0][t] = static_cast<float*>(tm.psi);
+      d.psi[1][t] = take(numel(*(t < 2 ? in.h.psi_in[t] : in.e.psi_in[t - 2])));
+    }
+  }
+  // sources: pre-E Ez, H-timed Hx and Hy, E-timed Ez
+  if (in.ngroups == 9) {
+    for (int gi : {0, 1, 5, 6, 7})
+      if (group_slabs(in.groups[gi]) > 0) return false;
+    if (!add_tm_slabs(d, in.groups[2], kEz, ez, false, in.metallic)) return false;
+    d.nslab_pre = d.nslab;
+    if (!add_tm_slabs(d, in.groups[3], kHx, hx, true, in.metallic)) return false;
+    if (!add_tm_slabs(d, in.groups[4], kHy, hy, true, in.metallic)) return false;
+    d.nslab_h = d.nslab;
+    if (!add_tm_slabs(d, in.groups[8], kEz, ez, true, in.metallic)) return false;
+  }
+  p.step0 = in.step ? static_cast<const int32_t*>(in.step->data) : nullptr;
+  if (d.nslab > 0 && p.step0 == nullptr) return false;
+  if (in.has_monitors) {
+    if (in.mon_boxes == nullptr || slots < 2) return false;
+    dc.d = make_dft(in.mon, in.bank_a, g, in.dt, in.monitor_count);
+    if (dc.d.M < 1 || dc.d.M > kMaxMonBoxes) return false;
+    const int32_t* hb = static_cast<const int32_t*>(in.mon_boxes->data);
+    int64_t cells = 0;
+    for (int m = 0; m < dc.d.M; ++m) {
+      for (int q = 0; q < 3; ++q) {
+        const int c = q == 2 ? 2 : q + 3;  // DFT order
+        TmBox& b = dc.box[m][q];
+        b = {1, 0, 1, 0, q, 0};
+        const int32_t* x = hb + (m * 6 + c) * 6;
+        if (x[0] < 0) continue;
+        BZH_REQUIRE(x[2] >= 0 && x[2] <= x[3] && x[3] < dc.d.fdims[c][1] && x[4] >= 0 &&
+                        x[4] <= x[5] && x[5] < dc.d.fdims[c][2],
+                    "monitor box " + std::to_string(m) + " lies outside component " + std::to_string(c));
+        b = {x[2], x[3], x[4], x[5], q, static_cast<int32_t>(cells)};
+        cells += static_cast<int64_t>(x[3] - x[2] + 1) * (x[5] - x[4] + 1);
+        if (cells >= (int64_t{1} << 26)) return false;
+        p.box[p.nbox++] = b;
+      }
+    }
+    p.cap_cells = dc.cap_cells = static_cast<int32_t>(std::max<int64_t>(cells, 1));
+    p.cap = take(int64_t{slots} * p.cap_cells);
+    dc.cap = p.cap;
+  }
+  if (in.record != nullptr) {
+    p.record = in.record->record;
+    for (int q = 0; q < 4; ++q) p.design[q] = in.record->design[q];
+  }
+  return used <= have;
+}
+
+// The launches of a 2D multi-step call: an even number of them, so that the
+// result lands in bank A, the steps dealt out evenly, and the captured DFT
+// folded whenever the next launch would overflow the capture's slots.
+void tm_schedule(const ProgramIn& in, const Grid& g, TmParams& p, DftCapParams& dc, int slots,
+                 std::vector<Launch>& launches) {
+  const TmShape shape = tm_shape(g.ny, g.nx);
+  const int T = in.has_monitors ? std::min(shape.T, slots) : shape.T;
+  const int n = std::max(2, (in.nsteps + 2 * T - 1) / (2 * T) * 2);
+  const int slot0 = in.record != nullptr ? in.record->slot : 0;
+  p.rpt = shape.rpt;
+  int k = 0, filled = 0;
+  for (int i = 0; i < n; ++i) {
+    p.T = in.nsteps / n + (i < in.nsteps % n ? 1 : 0);
+    p.k = k;
+    p.bank = i & 1;
+    p.ntx = (g.nx + 1 + 63 - 2 * p.T) / (64 - 2 * p.T);
+    p.cap_slot = filled;
+    p.record_slot = slot0 + k;
+    launches.push_back(make_launch(Kind::kTm, 0, g.dtype, p));
+    k += p.T;
+    filled += p.T;
+    const int next = i + 1 < n ? in.nsteps / n + (i + 1 < in.nsteps % n ? 1 : 0) : 0;
+    if (in.has_monitors && (i + 1 == n || filled + next > slots)) {
+      dc.d.nk = filled;
+      dc.d.k0 = k - filled;
+      launches.push_back(make_launch(Kind::kDftCapture, 0, g.dtype, dc));
+      filled = 0;
+    }
+  }
+}
+
 // Returns true when the fused two-bank kernel carried the whole schedule (psi
 // then ping-pongs with the fields); false for the per-phase schedule.
 bool run_program(hipStream_t s, ProgramIn& in) {
@@ -1423,6 +1650,18 @@ bool run_program(hipStream_t s, ProgramIn& in) {
                      (!cpml_probe.wide ||
                       (g.dtype == BZH_F32 && !cpml_probe.psi_bf16 && fused_rows() == 15));
   const int32_t* step0 = in.step ? static_cast<const int32_t*>(in.step->data) : nullptr;
+  if (!g.is3d) {
+    TmParams tp;
+    DftCapParams dc;
+    const int tm_slots = dft_slots(in.nsteps);
+    if (tm_program(in, g, tp, dc, tm_slots)) {
+      std::vector<Launch> launches;
+      tm_schedule(in, g, tp, dc, tm_slots, launches);
+      graph_cache().run(s, launches, (in.flags & BZH_FLAG_GRAPH_CACHE) != 0);
+      g_last_pairs = g_last_capture = g_last_fused = 0;
+      return false;
+    }
+  }
   int slots = 1;
   float* stage = nullptr;
   if (in.has_monitors) {
@@ -1726,6 +1965,12 @@ bool run_program(hipStream_t s, ProgramIn& in) {
       for (int c = 0; c < 3 && 6 + c < in.ngroups; ++c)
         add_source_launches(launches, in.groups[6 + c], 2, c, nxt, g, in.metallic, step0, k);
     if (in.has_monitors) add_dft(k, nxt);
+    if (in.record != nullptr) {
+      AdjointRecordParams rp{*in.record, static_cast<const float*>(nxt[kHx]->data),
+                             static_cast<const float*>(nxt[kHy]->data)};
+      rp.p.slot += k;
+      launches.push_back(make_launch(Kind::kAdjointRecord, 0, g.dtype, rp));
+    }
     cur_b = two_banks ? !cur_b : cur_b;
     ++k;
   }
@@ -1854,7 +2099,7 @@ int decode_program(const bzh_buffer* args, int nargs, const bzh_program_attrs& a
     in.step = in.mon.b[11];
     in.has_monitors = true;
     next += 12;
-    if (nargs == next + 1) {
+    if (nargs > next && (temporal || nargs > next + 1 || args[next].element_type == BZH_S32)) {
       const bzh_buffer* hb = arg(args, nargs, next++);
       BZH_REQUIRE(hb->element_type == BZH_S32 && numel(*hb) == 36 * in.monitor_count &&
                       (hb->data != nullptr || in.monitor_count == 0),
@@ -1862,6 +2107,10 @@ int decode_program(const bzh_buffer* args, int nargs, const bzh_program_attrs& a
       in.mon_boxes = hb;
     }
   }
+  // the in-place layouts' optional workspace, after any monitor boxes
+  if (!temporal && nargs == next + 1 && in.bank_a[kEz]->rank == 2 &&
+      args[next].element_type == BZH_F32 && args[next].rank == 1)
+    in.workspace = arg(args, nargs, next++);
   BZH_REQUIRE(next == nargs, "layout " + std::to_string(layout) + " expects " +
                                  std::to_string(next) + " arguments, got " + std::to_string(nargs));
   if (in.ngroups > 0) BZH_REQUIRE(in.step && in.step->element_type == BZH_S32,
@@ -2239,6 +2488,27 @@ int32_t bzh_adjoint2d_record(void* stream, const bzh_adjoint2d* adj, const bzh_b
     const float* fhx = f32_ptr(*hx, static_cast<int64_t>(p.ny) * (p.nx + 1), "forward Hx");
     const float* fhy = f32_ptr(*hy, static_cast<int64_t>(p.ny + 1) * p.nx, "forward Hy");
     launch_adjoint_record(static_cast<hipStream_t>(stream), p, fhx, fhy);
+  });
+}
+
+int32_t bzh_adjoint2d_recompute(void* stream, const bzh_buffer* args, int32_t nargs,
+                                const bzh_program_attrs* attrs, const bzh_adjoint2d* adj,
+                                int32_t slot) {
+  return guarded([&] {
+    BZH_REQUIRE(attrs != nullptr && args != nullptr && adj != nullptr, "null arguments");
+    BZH_REQUIRE(attrs->abi_version == BZH_ABI_VERSION, "ABI version mismatch");
+    ProgramIn in;
+    const int temporal = decode_program(args, nargs, *attrs, in);
+    BZH_REQUIRE(!temporal && in.bank_a[kEz]->rank == 2, "the recompute steps a 2D in-place program");
+    int64_t slots = 0;
+    Adjoint2dParams p = describe_adjoint(*adj, &slots);
+    BZH_REQUIRE(in.nsteps >= 1 && slot >= 0 && slot + in.nsteps <= slots, "record slots out of range");
+    const Grid g = infer_grid(in.bank_a);
+    BZH_REQUIRE(g.dtype == BZH_F32 && g.ny == p.ny && g.nx == p.nx,
+                "the recomputed program does not match the adjoint grid");
+    p.slot = slot;
+    in.record = &p;
+    run_program(static_cast<hipStream_t>(stream), in);
   });
 }
 

@@ -399,6 +399,23 @@ struct DftParams {
 constexpr int kDftMaxSlots = 32;
 void launch_dft(hipStream_t s, const DftParams& p);
 
+// The DFT of a 2D multi-step call: fold steps d.k0 .. d.k0 + d.nk - 1, whose
+// monitored cells sit in slots 0 .. nk - 1 of the capture, into the
+// accumulators.  box[m][q]: the captured box of monitor m's component Hx, Hy,
+// Ez (q 0, 1, 2); y0 > y1 when it is not gathered.
+struct TmBox {             // cells captured after every step (inclusive)
+  int32_t y0, y1, x0, x1;
+  int32_t comp;            // 0 Hx, 1 Hy, 2 Ez
+  int32_t off;             // first cell in a capture slot, row-major
+};
+struct DftCapParams {
+  DftParams d;
+  TmBox box[kMaxMonBoxes][3];
+  const float* cap;        // [slots][cap_cells]
+  int32_t cap_cells;
+};
+void launch_dft_capture(hipStream_t s, const DftCapParams& p);
+
 // One TMxy simulation of a batch on the device: two banks of (Ez, Hx, Hy),
 // uniform decays and H source, an E source array or scalar, CPML memories of
 // both banks (Hx_y, Hy_x, Ez_x, Ez_y), the coefficient table [4][3][2L] and
@@ -437,6 +454,57 @@ struct Batch2dParams {
 void launch_batch2d(hipStream_t s, const Batch2dParams& p);
 void launch_batch2d_sources(hipStream_t s, const Batch2dParams& p);
 
+// Several TMxy steps in one launch (tm_steps.hip): float32 fields and CPML
+// memories, scalar H coefficients, one CPML thickness L on every edge (0:
+// none), isotropic metrics.  Bank A (``_in``) is read, bank B written.
+constexpr int kTmMaxSteps = 8;
+constexpr int kTmRows = 32;   // rows of a tile (64 columns)
+constexpr int kMaxTmSlabs = 12;
+constexpr int kMaxTmBoxes = 3 * kMaxMonBoxes;
+struct TmSlab {            // a source slab, in order: pre-E, H-timed, E-timed
+  const float* coeff;      // [sz, sy, sx]
+  const float* wave;       // [T]
+  const int32_t* start;    // device int32[3]: (z, y, x); null: y0, x0 below
+  int32_t y0, x0;
+  int32_t sz, sy, sx, T;
+  int32_t comp;            // 0 Hx, 1 Hy, 2 Ez
+  int32_t fy, fx;          // the target's shape
+  int32_t mb, mt, ml, mr;  // PEC-constrained ends (post-update slabs)
+};
+struct TmSim {             // one simulation: bank a is read, bank 1 - a written
+  float* ez[2];
+  float* hx[2];
+  float* hy[2];
+  float* psi[2][4];        // Hx_y, Hy_x, Ez_x, Ez_y
+  const float* ta[4];      // their a, b, 1/kappa
+  const float* tb[4];
+  const float* tk[4];
+  const float* e_dec;      // per cell (dec_st 1) or a scalar, as e_src
+  const float* e_src;
+  const float* h_dec[2];   // scalars of Hx, Hy
+  const float* h_src[2];
+  int32_t dec_st, src_st;
+  float inv_dx;
+  int32_t ny, nx, L, metallic;
+  int32_t nslab, nslab_pre, nslab_h;   // [0, pre) pre-E, [pre, h) H, [h, n) E
+  TmSlab slab[kMaxTmSlabs];
+};
+struct TmParams {
+  TmSim sim;               // (first: the kernels re-read it from the argument block)
+  int32_t bank;            // bank read
+  int32_t T, k;            // steps of this launch, its first step in the call
+  const int32_t* step0;
+  int32_t rpt, ntx;        // rows per lane (2 or 4), tile columns
+  TmBox box[kMaxTmBoxes];
+  int32_t nbox;
+  float* cap;              // [slots][cap_cells]
+  int32_t cap_cells, cap_slot;
+  float* record;           // adjoint recompute: forward curl [K][dy][dx], or null
+  int32_t design[4];       // [y0, y1) x [x0, x1)
+  int32_t record_slot;
+};
+void launch_tm(hipStream_t s, const TmParams& p);
+
 // Reverse-time TMxy step (adjoint.hip).
 struct Adjoint2dParams {
   int32_t ny, nx, L, metallic;
@@ -464,6 +532,12 @@ struct Adjoint2dParams {
   double* grad;              // sum over steps of g * curl, [dy][dx]
 };
 void launch_adjoint_step(hipStream_t s, const Adjoint2dParams& p);
+// The record launch of one step, as a schedule entry.
+struct AdjointRecordParams {
+  Adjoint2dParams p;
+  const float* hx;
+  const float* hy;
+};
 void launch_adjoint_record(hipStream_t s, const Adjoint2dParams& p, const float* hx, const float* hy);
 
 

@@ -79,6 +79,13 @@ __device__ __forceinline__ float gather(const DftParams& p, int m, int c, int pt
   return v;
 }
 
+// sin and cos of 2 pi x for x turns.  Dropping whole turns first is exact and
+// spares sincos its reduction of arguments in the thousands, which took most
+// of a flush (the product f t carries the same relative rounding either way).
+__device__ __forceinline__ void phase_factor(double x, double& sn, double& cs) {
+  sincospi(2.0 * (x - rint(x)), &sn, &cs);
+}
+
 // Gate, window and amplitude factor of step k of this call for monitor m
 // (observe.py:315-357).  Returns false when the step is not sampled.
 __device__ __forceinline__ bool dft_gate(const DftParams& p, int m, int k, double& t,
@@ -119,87 +126,191 @@ __global__ void __launch_bounds__(kDftBlock) dft_stage_kernel(DftParams p) {
   p.stage[((slot * p.M + m) * 6 + c) * p.Pmax + pt] = gather<T>(p, m, c, pt);
 }
 
-// Buffered path: fold steps k0 .. k0+nk-1 of the ring into the accumulators.
-// Each step's term is formed exactly as in the direct path (f32 sample times
+// Fold steps k0 .. k0+nk-1 into the accumulators of frequencies f0 .. f0+kFt-1
+// (blockIdx.y picks the tile), given each step's gathered sample v[j].  A
+// step's term is formed exactly as in the direct path (f32 sample times
 // 1/scale, mask and amplitude in f64, times the f64 phase factor); the nk
 // terms of one (frequency, point) are summed in f64 and added once.
+constexpr int kFt = 8;
+struct FlushLds {
+  double t[kDftMaxSlots], scale[kDftMaxSlots], win[kDftMaxSlots];
+  int on[kDftMaxSlots];
+  double cs[kDftMaxSlots][kFt], sn[kDftMaxSlots][kFt];
+  float v[kDftMaxSlots][kDftBlock];  // each thread's samples (its own column)
+};
+// The steps' gates, the window sums and the phase factors of this block.
 template <typename A>
-__global__ void __launch_bounds__(kDftBlock) dft_flush_kernel(DftParams p) {
-  constexpr int kFt = 16;  // frequencies per LDS tile
-  const int m = blockIdx.z / 6;
-  const int c = blockIdx.z % 6;
-  const int P = p.counts[m * 5 + 1];
-  const int F = p.counts[m * 5 + 0];
-  const int64_t voff = p.counts[m * 5 + 3];
-  const int64_t woff = p.counts[m * 5 + 4];
+__device__ __forceinline__ void flush_begin(const DftParams& p, int m, int c, FlushLds& l) {
   const int nk = p.nk < kDftMaxSlots ? p.nk : kDftMaxSlots;
-  __shared__ double s_t[kDftMaxSlots], s_scale[kDftMaxSlots], s_win[kDftMaxSlots];
-  __shared__ int s_on[kDftMaxSlots];
-  __shared__ double s_cos[kDftMaxSlots][kFt], s_sin[kDftMaxSlots][kFt];
-  if (threadIdx.x < nk) {
+  const int F = p.counts[m * 5 + 0], nf = F < p.Fmax ? F : p.Fmax;
+  const int64_t woff = p.counts[m * 5 + 4];
+  const int f0 = blockIdx.y * kFt;
+  // this thread's frequency (its table entries e = threadIdx.x + i kDftBlock
+  // all have column e % kFt)
+  const int ft = f0 + static_cast<int>(threadIdx.x) % kFt;
+  double fr = 0.0;
+  if (ft < nf)
+    fr = p.freqs_f64 ? static_cast<const double*>(p.freqs)[m * p.Fmax + ft]
+                     : static_cast<double>(static_cast<const float*>(p.freqs)[m * p.Fmax + ft]);
+  if (threadIdx.x < kDftMaxSlots) {
     double t = 0.0, window = 0.0, scale = 0.0;
-    const bool on = dft_gate(p, m, p.k0 + threadIdx.x, t, window, scale);
-    s_t[threadIdx.x] = t;
-    s_scale[threadIdx.x] = on ? scale : 0.0;
-    s_win[threadIdx.x] = on ? window : 0.0;
-    s_on[threadIdx.x] = on ? 1 : 0;
+    const bool on = threadIdx.x < nk && dft_gate(p, m, p.k0 + threadIdx.x, t, window, scale);
+    l.t[threadIdx.x] = t;
+    l.scale[threadIdx.x] = on ? scale : 0.0;
+    l.win[threadIdx.x] = on ? window : 0.0;
+    l.on[threadIdx.x] = on ? 1 : 0;
   }
   __syncthreads();
-  const int nf = F < p.Fmax ? F : p.Fmax;
-  if (c == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
+  if (c == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
     A* w = static_cast<A*>(p.wsum);
-    for (int f = 0; f < nf; ++f) {
+    for (int f = threadIdx.x; f < nf; f += kDftBlock) {
       double acc = 0.0;
-      for (int j = 0; j < nk; ++j) acc += s_win[j];
+      for (int j = 0; j < nk; ++j) acc += l.win[j];
       if (woff + f < p.w_len) w[woff + f] += static_cast<A>(acc);
     }
   }
-  const float cmask = p.masks[m * 6 + c];
-  const int pt = blockIdx.x * kDftBlock + threadIdx.x;
-  const bool live = cmask != 0.0f && pt < P && pt < p.Pmax && p.field[c] != nullptr;
-  double dv[kDftMaxSlots];
+  static_assert(kDftBlock % kFt == 0, "a thread's entries share one frequency");
+  for (int e = threadIdx.x; e < kDftMaxSlots * kFt; e += kDftBlock) {
+    const int j = e / kFt;
+    double sn = 0.0, cs = 0.0;
+    if (ft < nf && j < nk) phase_factor(fr * l.t[j], sn, cs);
+    l.cs[j][e % kFt] = cs;
+    l.sn[j][e % kFt] = sn;
+  }
+  __syncthreads();
+}
+// The accumulators of (component, frequencies f0 .. f0 + kFt - 1, point),
+// loaded before the phase factors are formed: read one frequency after another
+// at the end, they were the kernel's longest chain.
+template <typename A>
+struct FlushAcc {
+  A re[kFt], im[kFt];
+  int64_t o;       // index of the first; frequency f sits P further per step
+  int P, n;        // n live frequencies (0: none)
+};
+template <typename A>
+__device__ __forceinline__ void flush_load(const DftParams& p, int m, int c, int pt, bool live,
+                                           FlushAcc<A>& a) {
+  const int P = p.counts[m * 5 + 1], F = p.counts[m * 5 + 0], nf = F < p.Fmax ? F : p.Fmax;
+  const int f0 = blockIdx.y * kFt;
+  a.P = P;
+  a.o = p.counts[m * 5 + 3] + (static_cast<int64_t>(c) * F + f0) * P + pt;
+  a.n = live ? max(0, min(kFt, nf - f0)) : 0;
 #pragma unroll
+  for (int f = 0; f < kFt; ++f) {
+    const int64_t o = a.o + static_cast<int64_t>(f) * P;
+    const bool in = f < a.n && o < p.re_len;
+    a.re[f] = in ? static_cast<const A*>(p.re)[o] : A(0);
+    a.im[f] = in ? static_cast<const A*>(p.im)[o] : A(0);
+  }
+}
+// (No step or frequency is skipped by a branch: steps past nk and frequencies
+// past the last carry zero factors, so that the reads and the 16 independent
+// sums pipeline.  The samples wait in LDS: with the step loop unrolled over a
+// register array the scheduler spilled.)
+template <typename A>
+__device__ __forceinline__ void flush_add(const DftParams& p, int m, int c, const FlushLds& l,
+                                          const FlushAcc<A>& acc) {
+  const float cmask = p.masks[m * 6 + c], inv = p.inv_scale[c];
+  double ar[kFt] = {}, ai[kFt] = {};
+#pragma unroll 2
   for (int j = 0; j < kDftMaxSlots; ++j) {
-    dv[j] = 0.0;
-    if (live && j < nk && s_on[j]) {
-      const int64_t slot = (p.k0 + j) % p.slots;
-      const float v = p.stage[((slot * p.M + m) * 6 + c) * p.Pmax + pt];
-      dv[j] = static_cast<double>(v) * p.inv_scale[c] * cmask * s_scale[j];
+    const double t = static_cast<double>(l.v[j][threadIdx.x]) * inv * cmask * l.scale[j];
+    const double dv = l.on[j] ? t : 0.0;
+#pragma unroll
+    for (int f = 0; f < kFt; ++f) {
+      ar[f] += dv * l.cs[j][f];
+      ai[f] += dv * l.sn[j][f];
     }
   }
   A* re = static_cast<A*>(p.re);
   A* im = static_cast<A*>(p.im);
-  for (int f0 = 0; f0 < nf; f0 += kFt) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < nk * kFt; e += kDftBlock) {
-      const int j = e / kFt, f = f0 + e % kFt;
-      double sn = 0.0, cs = 0.0;
-      if (f < nf) {
-        const double fr = p.freqs_f64 ? static_cast<const double*>(p.freqs)[m * p.Fmax + f]
-                                      : static_cast<double>(static_cast<const float*>(p.freqs)[m * p.Fmax + f]);
-        sincos(2.0 * M_PI * fr * s_t[j], &sn, &cs);
-      }
-      s_cos[j][e % kFt] = cs;
-      s_sin[j][e % kFt] = sn;
-    }
-    __syncthreads();
-    if (!live) continue;
-    for (int ff = 0; ff < kFt && f0 + ff < nf; ++ff) {
-      double ar = 0.0, ai = 0.0;
 #pragma unroll
-      for (int j = 0; j < kDftMaxSlots; ++j) {
-        if (j < nk) {
-          ar += dv[j] * s_cos[j][ff];
-          ai += dv[j] * s_sin[j][ff];
-        }
+  for (int f = 0; f < kFt; ++f) {
+    const int64_t o = acc.o + static_cast<int64_t>(f) * acc.P;
+    if (f < acc.n && o < p.re_len) {
+      re[o] = acc.re[f] + static_cast<A>(ar[f]);
+      im[o] = acc.im[f] + static_cast<A>(ai[f]);
+    }
+  }
+}
+
+// Buffered path: fold the ring's staged samples.  The frequency tiles are
+// separate blocks: 96 x 232-point planes of 11 frequencies took 108 us when
+// one block walked them all.
+template <typename A>
+__global__ void __launch_bounds__(kDftBlock) dft_flush_kernel(DftParams p) {
+  const int m = blockIdx.z / 6, c = blockIdx.z % 6;
+  const int P = p.counts[m * 5 + 1];
+  const int pt = blockIdx.x * kDftBlock + threadIdx.x;
+  const bool any = p.masks[m * 6 + c] != 0.0f && p.field[c] != nullptr;
+  if (!any && c != 0) return;  // (component 0 also adds the window sums)
+  const bool live = any && pt < P && pt < p.Pmax;
+  FlushAcc<A> acc;
+  flush_load<A>(p, m, c, pt, live, acc);
+  __shared__ FlushLds l;
+  flush_begin<A>(p, m, c, l);
+  if (!live) return;
+#pragma unroll 8
+  for (int j = 0; j < kDftMaxSlots; ++j) {
+    const int slot = (p.k0 + min(j, p.nk - 1)) % p.slots;
+    l.v[j][threadIdx.x] = p.stage[((static_cast<int64_t>(slot) * p.M + m) * 6 + c) * p.Pmax + pt];
+  }
+  flush_add<A>(p, m, c, l, acc);
+}
+
+// 2D multi-step calls: gather each step's sample from the captured cells and
+// fold it, without a launch per step.
+template <typename A>
+__global__ void __launch_bounds__(kDftBlock) dft_capture_kernel(DftCapParams p) {
+  const DftParams& d = p.d;
+  const int m = blockIdx.z / 6, c = blockIdx.z % 6;
+  const int P = d.counts[m * 5 + 1];
+  const int pt = blockIdx.x * kDftBlock + threadIdx.x;
+  const int q = c == 2 ? 2 : c - 3;  // (DFT order Ez 2, Hx 3, Hy 4)
+  const bool any = (c >= 2 && c <= 4) && d.masks[m * 6 + c] != 0.0f && d.field[c] != nullptr;
+  if (!any && c != 0) return;
+  // (the gather's loads, four corners at a time, are issued before the phase
+  // factors are formed: one corner after another behind them took 32 us for
+  // two 180-point lines)
+  float v[kDftMaxSlots];
+#pragma unroll
+  for (int j = 0; j < kDftMaxSlots; ++j) v[j] = 0.0f;
+  const bool live = any && pt < P && pt < d.Pmax;
+  FlushAcc<A> acc;
+  flush_load<A>(d, m, c, pt, live, acc);
+  if (live) {
+    const TmBox b = p.box[m][q];
+    const int64_t base = ((static_cast<int64_t>(m) * 6 + c) * d.Pmax + pt) * d.K;
+    const int sx = d.fdims[c][2];
+    for (int e0 = 0; e0 < d.K; e0 += 4) {
+      int idx[4];
+      float w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool in = e0 + e < d.K;
+        idx[e] = in ? d.indices[base + e0 + e] : -1;
+        w[e] = in ? d.weights[base + e0 + e] : 0.0f;
       }
-      const int64_t o = voff + (static_cast<int64_t>(c) * F + f0 + ff) * P + pt;
-      if (o < p.re_len) {
-        re[o] += static_cast<A>(ar);
-        im[o] += static_cast<A>(ai);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int y = idx[e] / sx, x = idx[e] - y * sx;
+        if (w[e] == 0.0f || idx[e] < 0 || idx[e] >= d.fsize[c] || y < b.y0 || y > b.y1 || x < b.x0 ||
+            x > b.x1)
+          continue;
+        const float* cell = p.cap + b.off + (y - b.y0) * (b.x1 - b.x0 + 1) + (x - b.x0);
+#pragma unroll
+        for (int j = 0; j < kDftMaxSlots; ++j)
+          v[j] += w[e] * cell[static_cast<int64_t>(min(j, d.nk - 1)) * p.cap_cells];
       }
     }
   }
+  __shared__ FlushLds l;
+#pragma unroll
+  for (int j = 0; j < kDftMaxSlots; ++j) l.v[j][threadIdx.x] = v[j];
+  flush_begin<A>(d, m, c, l);
+  if (!live) return;
+  flush_add<A>(d, m, c, l, acc);
 }
 
 template <typename T, typename A>
@@ -238,7 +349,7 @@ __global__ void __launch_bounds__(kDftBlock) dft_kernel(DftParams p) {
     const double fr = p.freqs_f64 ? static_cast<const double*>(p.freqs)[m * p.Fmax + f]
                                   : static_cast<double>(static_cast<const float*>(p.freqs)[m * p.Fmax + f]);
     double sn, cs;
-    sincos(2.0 * M_PI * fr * t, &sn, &cs);
+    phase_factor(fr * t, sn, cs);
     s_cos[f] = cs;
     s_sin[f] = sn;
   }
@@ -272,6 +383,7 @@ void dft_dispatch(hipStream_t s, const DftParams& p) {
   if (p.mode == 1) {
     hipLaunchKernelGGL((dft_stage_kernel<T>), grid, block, 0, s, p);
   } else if (p.mode == 2) {
+    grid.y = (p.Fmax + kFt - 1) / kFt;
     if (p.acc_f64) hipLaunchKernelGGL((dft_flush_kernel<double>), grid, block, 0, s, p);
     else hipLaunchKernelGGL((dft_flush_kernel<float>), grid, block, 0, s, p);
   } else {
@@ -371,6 +483,19 @@ void launch_dft(hipStream_t s, const DftParams& p) {
   BZH_HIP(hipGetLastError());
 }
 
+
+void launch_dft_capture(hipStream_t s, const DftCapParams& p) {
+  const DftParams& d = p.d;
+  if (d.M <= 0 || d.Pmax <= 0) return;
+  BZH_REQUIRE(d.Fmax <= kMaxFreq, "DFT monitors support at most 256 frequencies");
+  BZH_REQUIRE(d.M <= kMaxMonBoxes && d.nk >= 1 && d.nk <= kDftMaxSlots && p.cap != nullptr,
+              "captured DFT is malformed");
+  const dim3 block(kDftBlock),
+      grid((d.Pmax + kDftBlock - 1) / kDftBlock, (d.Fmax + kFt - 1) / kFt, d.M * 6);
+  if (d.acc_f64) hipLaunchKernelGGL((dft_capture_kernel<double>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((dft_capture_kernel<float>), grid, block, 0, s, p);
+  BZH_HIP(hipGetLastError());
+}
 
 void launch_monbox(hipStream_t s, const MonBoxParams& p) {
   BZH_REQUIRE(p.M >= 1 && p.M <= kMaxMonBoxes && p.box != nullptr, "monitor boxes are malformed");

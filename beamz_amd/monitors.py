@@ -386,17 +386,18 @@ def capture_boxes(idx, wts, masks, shapes):
     weight whose index lies inside the component (the kernels' gather rule),
     in the DFT component order Ex, Ey, Ez, Hx, Hy, Hz.  A component that no
     gather reads (mask zero or no live corner) has the row -1.  The pair
-    kernel captures exactly these cells of both its steps, so that the
-    monitors' samples are gathered from a dense buffer instead of strided
-    field rows (no counterpart in the reference, which samples every step
+    kernel captures exactly these cells of its first step, and the 2D
+    multi-step kernel those of every step, so that the monitors' samples are
+    gathered from a dense buffer instead of strided field rows (no counterpart in the reference, which samples every step
     from the fields)."""
     M = idx.shape[0]
     out = np.full((M, 6, 6), -1, dtype=np.int32)
     for m in range(M):
         for c, name in enumerate(COMPONENTS):
             shape = shapes.get(name)
-            if shape is None or len(shape) != 3 or masks[m, c] == 0.0:
+            if shape is None or masks[m, c] == 0.0:
                 continue
+            shape = (1,) * (3 - len(shape)) + tuple(shape)    # a 2D component is plane z = 0
             i = idx[m, c].reshape(-1).astype(np.int64)
             w = wts[m, c].reshape(-1)
             live = (w != 0.0) & (i >= 0) & (i < int(np.prod(shape)))

@@ -174,6 +174,9 @@ SIGNATURES = {
     "bzh_adjoint2d_record": (ctypes.c_int32, [ctypes.c_void_p, ctypes.POINTER(Adjoint2d),
                                               ctypes.POINTER(Buffer), ctypes.POINTER(Buffer),
                                               ctypes.c_int32]),
+    "bzh_adjoint2d_recompute": (ctypes.c_int32, [ctypes.c_void_p, ctypes.POINTER(Buffer),
+                                                 ctypes.c_int32, ctypes.POINTER(ProgramAttrs),
+                                                 ctypes.POINTER(Adjoint2d), ctypes.c_int32]),
     "bzh_adjoint2d_reverse": (ctypes.c_int32, [ctypes.c_void_p, ctypes.POINTER(Adjoint2d),
                                                ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
                                                ctypes.c_int32]),
@@ -302,6 +305,16 @@ class PreparedProgram:
         lib = library()
         s = current_stream_handle() if stream is None else stream
         _check(lib.bzh_program(s, self._arr, len(self._args), ctypes.byref(self._attrs)), lib)
+
+    def recompute(self, adj, nsteps, slot, stream=None):
+        """The call for ``nsteps`` steps that also records each step's forward
+        curl of ``adj`` from record slot ``slot`` (``bzh_adjoint2d_recompute``)."""
+        lib = library()
+        s = current_stream_handle() if stream is None else stream
+        attrs = ProgramAttrs.from_buffer_copy(self._attrs)
+        attrs.nsteps = int(nsteps)
+        _check(lib.bzh_adjoint2d_recompute(s, self._arr, len(self._args), ctypes.byref(attrs),
+                                           ctypes.byref(adj), int(slot)), lib)
 
 
 def call_batch2d(sims, current_step, attrs: BatchAttrs, stream=None):

@@ -90,9 +90,12 @@ class CompiledProgram:
     h_metrics: tuple = ()
     e_metrics: tuple = ()
     cell_grid: object = None       # the RectilinearGrid, or None for a uniform grid
-    # host s32[M, 6, 6] bounding boxes of the cells the monitors gather (3D),
-    # handed to the program as its optional trailing argument
+    # host s32[M, 6, 6] bounding boxes of the cells the monitors gather, handed
+    # to the program as its optional trailing argument
     monitor_boxes: torch.Tensor = None
+    # floats of the workspace that lets a 2D program run several steps per
+    # launch (0: it runs the per-phase schedule)
+    workspace_floats: int = 0
 
     @property
     def cells(self) -> int:
@@ -367,8 +370,7 @@ def compile_program(permittivity, resolution, dt, *, boundaries=(), sources=(), 
         packed = (_dev(idx, device, torch.int32), _dev(wts, device), _dev(fr, device, torch.float64),
                   _dev(masks, device), _dev(counts, device, torch.int32),
                   _dev(codes, device, torch.int32), _dev(windows, device))
-        if is_3d:
-            boxes = torch.from_numpy(capture_boxes(idx, wts, masks, shapes))
+        boxes = torch.from_numpy(capture_boxes(idx, wts, masks, shapes))
 
     return CompiledProgram(
         grid=grid, is_3d=is_3d, resolution=float(resolution), dt=float(dt), t0=float(t0),
@@ -379,9 +381,40 @@ def compile_program(permittivity, resolution, dt, *, boundaries=(), sources=(), 
         h_term_arrays=h_arrays, e_term_arrays=e_arrays, source_groups=groups,
         coincident_mask=coincident, monitors=compiled, packed_monitors=packed,
         monitor_boxes=boxes,
+        workspace_floats=0 if is_3d else workspace_floats_2d(shapes, cpml, field_dtype, psi_dtype,
+                                                             metric_kind, boxes),
         device=device, field_dtype=field_dtype, psi_dtype=psi_dtype, flags=int(flags), eps_cells=eps,
         eps_site=eps_site, metric_kind=metric_kind, h_metrics=h_metrics, e_metrics=e_metrics,
         cell_grid=cell_grid if metric_kind else None)
+
+
+# steps of captured monitor cells a 2D workspace holds (kDftMaxSlots of the
+# library) and the most cells per step it captures; programs whose monitors
+# read more run the per-phase schedule
+CAPTURE_SLOTS = 32
+MAX_CAPTURE_CELLS = 1 << 20
+
+
+def workspace_floats_2d(shapes, cpml, field_dtype, psi_dtype, metric_kind, boxes):
+    """Floats of a 2D program's multi-step workspace (``bzh_program``): a
+    second bank of the fields and CPML memories, each rounded up to 64 floats,
+    and 32 steps of the monitored cells; 0 where the library takes the
+    per-phase schedule anyway."""
+    if field_dtype != torch.float32 or psi_dtype != torch.float32 or metric_kind:
+        return 0
+    sizes = [int(np.prod(s)) for s in shapes.values()]
+    for t in (cpml.h_terms + cpml.e_terms) if cpml is not None else ():
+        shape = list(shapes[t.component])
+        shape[t.axis] = t.low + t.high
+        sizes.append(int(np.prod(shape)))
+    if boxes is not None:
+        b = boxes.numpy().astype(np.int64)
+        ext = b[..., 1::2] - b[..., ::2] + 1
+        cells = int(np.sum(np.prod(ext, axis=-1) * (b[..., 0] >= 0)))
+        if cells > MAX_CAPTURE_CELLS:
+            return 0
+        sizes.append(CAPTURE_SLOTS * max(cells, 1))
+    return sum(-(-n // 64) * 64 for n in sizes)
 
 
 def _lower_metrics(cell_grid, grid, is_3d, device):

@@ -161,13 +161,28 @@ def _temporal_io(prog, state):
     return (*_graph_io(prog, state), *state.fields_b)
 
 
+def with_workspace_2d(state, prog):
+    """The state with the 2D program's multi-step workspace in its second-bank
+    slot (allocated on first use; its contents do not outlive a call)."""
+    n = prog.workspace_floats
+    if n == 0 or prog.is_3d or (len(state.fields_b) == 1 and state.fields_b[0].numel() >= n):
+        return state
+    return state._replace(fields_b=(torch.empty(n, dtype=torch.float32, device=prog.device),))
+
+
+def _workspace_args(state, prog):
+    return tuple(state.fields_b[:1]) if prog.workspace_floats and not prog.is_3d else ()
+
+
 def run_steps(state, prog, nsteps):
     """Source-free, monitor-free steps (``runtime.py:685-750``).  Returns the
     state holding the result (the bank roles swap after an odd count)."""
     if uses_two_banks(prog):
         return run_source_group_steps(state, prog, nsteps)
     layout = abi.PROGRAM_LAYOUT_CPML_IN_PLACE if prog.cpml_enabled else abi.PROGRAM_LAYOUT_YEE_IN_PLACE
-    native.call_program(_graph_io(prog, state), _program_attrs(prog, nsteps, layout))
+    state = with_workspace_2d(state, prog)
+    native.call_program((*_graph_io(prog, state), *_workspace_args(state, prog)),
+                        _program_attrs(prog, nsteps, layout))
     return state
 
 
@@ -180,7 +195,9 @@ def run_source_group_steps(state, prog, nsteps, *, noalloc=False):
         native.call_program(args, _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_SOURCE_TEMPORAL_CPML),
                             noalloc=noalloc)
         return _swap_banks(state, nsteps)
-    args = (*_graph_io(prog, state), *_source_group_arguments(prog), state.current_step)
+    state = state if noalloc else with_workspace_2d(state, prog)
+    args = (*_graph_io(prog, state), *_source_group_arguments(prog), state.current_step,
+            *_workspace_args(state, prog))
     native.call_program(args, _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_SOURCE_IN_PLACE),
                         noalloc=noalloc)
     return state
@@ -209,7 +226,8 @@ def run_program_steps(state, prog, nsteps, *, noalloc=False):
                             _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_MONITOR_TEMPORAL_CPML,
                                            monitor_count=len(prog.monitors)), noalloc=noalloc)
         return _swap_banks(state, nsteps)
-    native.call_program((*_graph_io(prog, state), *tail),
+    state = state if noalloc else with_workspace_2d(state, prog)
+    native.call_program((*_graph_io(prog, state), *tail, *_workspace_args(state, prog)),
                         _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_MONITOR_IN_PLACE,
                                        monitor_count=len(prog.monitors)), noalloc=noalloc)
     return state
@@ -233,17 +251,19 @@ def prepare_chunk(state, prog, nsteps):
     None for a program that steps through two banks."""
     if uses_two_banks(prog):
         return None
+    state = with_workspace_2d(state, prog)
+    ws = _workspace_args(state, prog)
     if prog.monitors:
         return native.PreparedProgram(
-            (*_graph_io(prog, state), *_monitor_tail(state, prog, False)),
+            (*_graph_io(prog, state), *_monitor_tail(state, prog, False), *ws),
             _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_MONITOR_IN_PLACE,
                            monitor_count=len(prog.monitors)))
     if any(g is not None for g in prog.source_groups):
         return native.PreparedProgram(
-            (*_graph_io(prog, state), *_source_group_arguments(prog), state.current_step),
+            (*_graph_io(prog, state), *_source_group_arguments(prog), state.current_step, *ws),
             _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_SOURCE_IN_PLACE))
     layout = abi.PROGRAM_LAYOUT_CPML_IN_PLACE if prog.cpml_enabled else abi.PROGRAM_LAYOUT_YEE_IN_PLACE
-    return native.PreparedProgram(_graph_io(prog, state), _program_attrs(prog, nsteps, layout))
+    return native.PreparedProgram((*_graph_io(prog, state), *ws), _program_attrs(prog, nsteps, layout))
 
 
 GRAPH_MAX_STEPS = 256  # execute.py:64

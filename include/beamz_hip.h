@@ -226,7 +226,12 @@ int32_t bzh_streamed(void* stream, const bzh_buffer* args, int32_t nargs,
  * s32[M, 6, 6] inclusive boxes (z0, z1, y0, y1, x0, x1; -1 when unused) of
  * the cells each monitor gathers per component (Ex, Ey, Ez, Hx, Hy, Hz).
  * With it, two-step launches capture those cells densely instead of writing
- * an intermediate bank; results are the same. */
+ * an intermediate bank; results are the same.  The in-place layouts (0, 2, 3
+ * and 5) of a 2D (TMxy) program take one more optional last argument, an f32
+ * device workspace (rank 1): with room for a second bank of Ez, Hx, Hy and the
+ * four CPML memories, each rounded up to 64 floats, and for 32 steps of the
+ * boxes' cells, float32 programs run several steps per launch; the results
+ * are bitwise the same and the workspace's contents are undefined after. */
 int32_t bzh_program(void* stream, const bzh_buffer* args, int32_t nargs,
                     const bzh_program_attrs* attrs);
 
@@ -315,6 +320,12 @@ typedef struct bzh_adjoint2d {
  * record[slot]; call after each forward step of a recomputed segment. */
 int32_t bzh_adjoint2d_record(void* stream, const bzh_adjoint2d* adj, const bzh_buffer* hx,
                              const bzh_buffer* hy, int32_t slot);
+/* A 2D in-place program of attrs->nsteps steps (args and attrs as bzh_program)
+ * that records the forward curl of its step k into record[slot + k]: the
+ * recompute of a checkpoint segment in one call. */
+int32_t bzh_adjoint2d_recompute(void* stream, const bzh_buffer* args, int32_t nargs,
+                                const bzh_program_attrs* attrs, const bzh_adjoint2d* adj,
+                                int32_t slot);
 /* Reverse forward steps n_last, n_last-1, ..., n_last-count+1, whose curls
  * sit in record slots slot_last, slot_last-1, ...  flags: BZH_FLAG_GRAPH_CACHE. */
 int32_t bzh_adjoint2d_reverse(void* stream, const bzh_adjoint2d* adj, int32_t n_last,
