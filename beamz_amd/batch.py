@@ -1,18 +1,17 @@
-"""Many independent 2D (TMxy) simulations in one persistent launch per step.
+"""Many independent 2D (TMxy) simulations in one launch per several steps.
 
 The reference runs one simulation per call and vmaps its FFI sequentially
 (``beamz/simulation/cuda/runtime.py:85``); parameter sweeps and optimizer
 populations therefore pay one launch chain per simulation.  Here every
-simulation of a batch is cut into 62-column items, the items of all
-simulations form one list, and the waves of one grid take them round-robin
--- one march launch per time step for the whole batch (after a small launch
-that adds the step's pre-E sources), uneven grid sizes included.  A chunk
-of up to 256 steps is captured once as a hipGraph and replayed.
+simulation of a batch is cut into tiles, the tiles of all simulations form one
+grid, and a launch advances all of them up to eight steps (temporal blocking,
+``csrc/tm_steps.hip``), uneven grid sizes included.  A chunk of up to 256 steps
+is captured once as a hipGraph and replayed.
 
 Each member is lowered exactly like a single simulation (``program.py``):
 same coefficients, CPML profiles, PEC faces and pre-E soft sources, so a
-member of a batch reproduces the same simulation run alone.  The tile height
-and the grid size are chosen by :func:`autotune` on the actual batch.
+member of a batch reproduces the same simulation run alone.  The rows a lane
+holds (``tile_rows``) are chosen by :func:`autotune` on the actual batch.
 """
 
 from __future__ import annotations
@@ -28,7 +27,9 @@ from . import native
 from .api import Simulation
 from .program import CompiledProgram
 
-TILE_ROWS = (8, 16, 32, 64)
+# 16: two rows per lane (16-wave tiles: fewer tiles than CUs), 32: four (8 and
+# 64 are taken as these)
+TILE_ROWS = (16, 32)
 MAX_SOURCES = 4
 _TUNED: dict = {}
 
@@ -213,21 +214,17 @@ class BatchedSimulation2D:
 
 
 def autotune(batch: BatchedSimulation2D, *, steps=6, candidates=None, verbose=False):
-    """Pick the tile height and persistent grid size of ``batch`` by timing
-    each candidate for a few steps on a scratch state; the choice is cached
-    per batch signature (grid shapes and CPML thickness).  Returns
-    ``(tile_rows, workgroups, timings)``."""
+    """Pick ``tile_rows`` of ``batch`` by timing each candidate for a few steps
+    on a scratch state; the choice is cached per batch signature (grid shapes
+    and CPML thickness).  Returns ``(tile_rows, workgroups, timings)``; every
+    tile is its own workgroup, so ``workgroups`` changes nothing."""
     steps = max(2, steps + steps % 2)  # even: the banks end where they start
     key = batch.signature()
     if key in _TUNED:
         batch.tile_rows, batch.workgroups = _TUNED[key][:2]
         return _TUNED[key]
-    props = torch.cuda.get_device_properties(batch.progs[0].device)
-    cus = int(props.multi_processor_count)
     if candidates is None:
-        # (64 and 96 workgroups per CU measured 1.3-1.5 % faster than 32 on the
-        # 64-simulation sweep at 8 rows)
-        candidates = [(tr, wg * cus) for tr in TILE_ROWS for wg in (8, 16, 32, 64, 96)]
+        candidates = [(tr, 0) for tr in TILE_ROWS]
     scratch = batch.initial_state()
     timings = {}
     stream = torch.cuda.current_stream()

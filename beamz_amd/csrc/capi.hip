@@ -387,10 +387,9 @@ void enqueue(hipStream_t s, const Launch& l) {
       break;
     }
     case Kind::kBatch2d: {
-      Batch2dParams p;
+      TmBatchParams p;
       std::memcpy(&p, l.bytes.data(), sizeof(p));
-      if (l.phase == 1) launch_batch2d_sources(s, p);
-      else launch_batch2d(s, p);
+      launch_tm_batch(s, p);
       break;
     }
     case Kind::kAdjoint: {
@@ -1393,11 +1392,13 @@ bool metrics_empty(const PhaseIn& ph) {
 struct TmShape {
   int T, rpt;
 };
+int tm_steps_per_launch(int64_t tiles) {
+  if (const char* env = std::getenv("BZH_TM_T")) return std::max(2, std::min(std::atoi(env), kTmMaxSteps));
+  return tiles <= 2048 ? 8 : 6;
+}
 TmShape tm_shape(int ny, int nx) {
   const int64_t tiles = int64_t{(nx + 48) / 48} * ((ny + 16) / 16);
-  TmShape t{tiles <= 2048 ? 8 : 6, tiles <= 256 ? 2 : 4};
-  if (const char* env = std::getenv("BZH_TM_T")) t.T = std::max(2, std::min(std::atoi(env), kTmMaxSteps));
-  return t;
+  return {tm_steps_per_launch(tiles), tiles <= 256 ? 2 : 4};
 }
 
 // The source slabs of group gi (E components of ``timing`` 0 or 2, H of 1).
@@ -2161,9 +2162,9 @@ float* f32_ptr(const bzh_buffer& b, int64_t expect, const std::string& what) {
 }
 
 
-Sim2dDev describe_sim2d(const bzh_sim2d& in, int index) {
+TmSim describe_sim2d(const bzh_sim2d& in, int index) {
   const std::string who = "simulation " + std::to_string(index) + ": ";
-  Sim2dDev d;
+  TmSim d;
   std::memset(&d, 0, sizeof(d));
   BZH_REQUIRE(in.ez[0].rank == 2, who + "Ez must be rank 2");
   d.ny = static_cast<int>(in.ez[0].dims[0]) - 1;
@@ -2181,41 +2182,70 @@ Sim2dDev describe_sim2d(const bzh_sim2d& in, int index) {
   BZH_REQUIRE(d.ez[0] != d.ez[1] && d.hx[0] != d.hx[1] && d.hy[0] != d.hy[1],
               who + "the two field banks must be distinct");
   d.e_dec = f32_ptr(in.e_decay, 1, who + "E decay");
-  d.h_dec = f32_ptr(in.h_decay, 1, who + "H decay");
-  d.h_src = f32_ptr(in.h_source, 1, who + "H source");
-  d.e_src_st = numel(in.e_source) == 1 ? 0 : 1;
-  d.e_src = f32_ptr(in.e_source, d.e_src_st ? nez : 1, who + "E source");
+  d.h_dec[0] = d.h_dec[1] = f32_ptr(in.h_decay, 1, who + "H decay");
+  d.h_src[0] = d.h_src[1] = f32_ptr(in.h_source, 1, who + "H source");
+  d.src_st = numel(in.e_source) == 1 ? 0 : 1;
+  d.e_src = f32_ptr(in.e_source, d.src_st ? nez : 1, who + "E source");
   BZH_REQUIRE(in.resolution > 0.0f, who + "resolution must be positive");
   d.inv_dx = 1.0f / in.resolution;
   d.metallic = in.metallic & (kBottom | kTop | kLeft | kRight);
   d.L = in.cpml_cells;
   BZH_REQUIRE(d.L >= 0 && 2 * d.L <= std::min(d.ny, d.nx), who + "CPML thicker than the grid");
+  // (a member without CPML reads entry 0 of its coefficient rows and uses none)
+  for (int t = 0; t < 4; ++t) d.ta[t] = d.tb[t] = d.tk[t] = d.h_dec[0];
   if (d.L > 0) {
     const int64_t L2 = 2 * d.L;
-    d.tab = f32_ptr(in.cpml_table, 12 * L2, who + "CPML table");
+    const float* tab = f32_ptr(in.cpml_table, 12 * L2, who + "CPML table");
     const int64_t sizes[4] = {L2 * (d.nx + 1), (d.ny + 1) * L2, (d.ny + 1) * L2, L2 * (d.nx + 1)};
-    for (int b = 0; b < 2; ++b)
-      for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < 4; ++t) {
+      d.ta[t] = tab + (3 * t + 0) * L2;
+      d.tb[t] = tab + (3 * t + 1) * L2;
+      d.tk[t] = tab + (3 * t + 2) * L2;
+      for (int b = 0; b < 2; ++b)
         d.psi[b][t] = f32_ptr(in.psi[b][t], sizes[t], who + "CPML memory " + std::to_string(t));
+    }
   }
   BZH_REQUIRE(in.nsrc >= 0 && in.nsrc <= 4, who + "at most four sources");
-  d.nsrc = in.nsrc;
+  d.nslab = d.nslab_pre = d.nslab_h = in.nsrc;
   for (int q = 0; q < in.nsrc; ++q) {
     const bzh_buffer& c = in.src_coeff[q];
     BZH_REQUIRE(c.rank == 2, who + "source coefficients must be (sy, sx)");
-    d.src_sy[q] = static_cast<int>(c.dims[0]);
-    d.src_sx[q] = static_cast<int>(c.dims[1]);
-    d.src_y0[q] = in.src_start[q][0];
-    d.src_x0[q] = in.src_start[q][1];
-    BZH_REQUIRE(d.src_y0[q] >= 0 && d.src_x0[q] >= 0 && d.src_y0[q] + d.src_sy[q] <= d.ny + 1 &&
-                    d.src_x0[q] + d.src_sx[q] <= d.nx + 1,
+    TmSlab& s = d.slab[q];
+    s.sz = 1;
+    s.sy = static_cast<int>(c.dims[0]);
+    s.sx = static_cast<int>(c.dims[1]);
+    s.y0 = in.src_start[q][0];
+    s.x0 = in.src_start[q][1];
+    BZH_REQUIRE(s.y0 >= 0 && s.x0 >= 0 && s.y0 + s.sy <= d.ny + 1 && s.x0 + s.sx <= d.nx + 1,
                 who + "source slab leaves the Ez support");
-    d.src_coeff[q] = f32_ptr(c, static_cast<int64_t>(d.src_sy[q]) * d.src_sx[q], who + "source coefficients");
-    d.src_T[q] = static_cast<int>(numel(in.src_wave[q]));
-    BZH_REQUIRE(d.src_T[q] >= 1, who + "source waveform is empty");
-    d.src_wave[q] = f32_ptr(in.src_wave[q], d.src_T[q], who + "source waveform");
+    s.coeff = f32_ptr(c, static_cast<int64_t>(s.sy) * s.sx, who + "source coefficients");
+    s.T = static_cast<int>(numel(in.src_wave[q]));
+    BZH_REQUIRE(s.T >= 1, who + "source waveform is empty");
+    s.wave = f32_ptr(in.src_wave[q], s.T, who + "source waveform");
+    s.comp = 2;
+    s.fy = d.ny + 1;
+    s.fx = d.nx + 1;
   }
   return d;
+}
+
+// The tiles of every member at T steps per launch, largest simulations first,
+// row-major within one.
+std::vector<int4> batch_tiles(const std::vector<TmSim>& sims, int T) {
+  std::vector<int> order(sims.size());
+  for (size_t i = 0; i < order.size(); ++i) order[i] = static_cast<int>(i);
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+    return static_cast<int64_t>(sims[x].ny) * sims[x].nx > static_cast<int64_t>(sims[y].ny) * sims[y].nx;
+  });
+  const int cols = 64 - 2 * T, rows = kTmRows - 2 * T;
+  std::vector<int4> tiles;
+  for (int i : order) {
+    const int ty = (sims[i].ny + rows) / rows, tx = (sims[i].nx + cols) / cols;
+    for (int r = 0; r < ty; ++r)
+      for (int c = 0; c < tx; ++c) tiles.push_back(make_int4(i, r, c, 0));
+  }
+  BZH_REQUIRE(tiles.size() < (size_t{1} << 31), "too many tiles");
+  return tiles;
 }
 
 void run_batch2d(hipStream_t s, const bzh_sim2d* sims, int nsims, const bzh_buffer* step,
@@ -2226,47 +2256,36 @@ void run_batch2d(hipStream_t s, const bzh_sim2d* sims, int nsims, const bzh_buff
               "tile_rows must be 8, 16, 32 or 64");
   BZH_REQUIRE(step != nullptr && step->element_type == BZH_S32 && step->data && numel(*step) == 1,
               "current_step must be an s32 scalar");
-  std::vector<Sim2dDev> desc(nsims);
-  for (int i = 0; i < nsims; ++i) desc[i] = describe_sim2d(sims[i], i);
-  // queue: largest simulations first, row-major items (62 columns by
-  // tile_rows rows) within one
-  std::vector<int> order(nsims);
-  for (int i = 0; i < nsims; ++i) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-    return static_cast<int64_t>(desc[x].ny) * desc[x].nx > static_cast<int64_t>(desc[y].ny) * desc[y].nx;
-  });
-  std::vector<int4> tiles;
-  for (int i : order) {
-    const int ty = (desc[i].ny + 1 + a.tile_rows - 1) / a.tile_rows, tx = (desc[i].nx + 1 + 61) / 62;
-    for (int r = 0; r < ty; ++r)
-      for (int c = 0; c < tx; ++c) tiles.push_back(make_int4(i, r, c, 0));
+  std::vector<TmSim> desc(nsims);
+  int64_t tiles = 0;
+  for (int i = 0; i < nsims; ++i) {
+    desc[i] = describe_sim2d(sims[i], i);
+    tiles += int64_t{(desc[i].nx + 48) / 48} * ((desc[i].ny + 16) / 16);
   }
-  BZH_REQUIRE(tiles.size() < (size_t{1} << 31), "too many tiles");
-  int workgroups = a.workgroups;
-  if (workgroups <= 0) {
-    int device = 0, cus = 0;
-    BZH_HIP(hipGetDevice(&device));
-    BZH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-    workgroups = 4 * std::max(cus, 1);
-  }
-  Batch2dParams p;
+  const int T = tm_steps_per_launch(tiles);
+  // as many launches as keep the single-step bank parity: the result is in
+  // bank 1 after an odd step count
+  int n = (a.nsteps + T - 1) / T;
+  if ((a.nsteps - n) % 2 != 0) ++n;
+  TmBatchParams p;
   std::memset(&p, 0, sizeof(p));
-  p.sims = static_cast<const Sim2dDev*>(upload_cached(desc));
-  p.tiles = static_cast<const int4*>(upload_cached(tiles));
-  p.ntiles = static_cast<int>(tiles.size());
+  p.sims = static_cast<const TmSim*>(upload_cached(desc));
   p.step0 = static_cast<const int32_t*>(step->data);
-  p.tile_rows = a.tile_rows;
-  p.workgroups = workgroups;
-  p.nsims = nsims;
-  for (const Sim2dDev& d : desc)
-    for (int q = 0; q < d.nsrc; ++q) p.max_src_cells = std::max(p.max_src_cells, d.src_sy[q] * d.src_sx[q]);
+  p.rpt = a.tile_rows <= 16 ? 2 : 4;
   std::vector<Launch> launches;
-  for (int k = 0; k < a.nsteps; ++k) {
-    p.k = k;
-    p.bank = k & 1;
-    // the step's pre-E sources on the bank it reads, then the march
-    if (p.max_src_cells > 0) launches.push_back(make_launch(Kind::kBatch2d, 1, BZH_F32, p));
+  int done = 0;
+  for (int i = 0; i < n; ++i) {
+    const int steps = a.nsteps / n + (i < a.nsteps % n ? 1 : 0);
+    if (steps != p.T) {
+      const std::vector<int4> list = batch_tiles(desc, steps);
+      p.tiles = static_cast<const int4*>(upload_cached(list));
+      p.ntiles = static_cast<int>(list.size());
+      p.T = steps;
+    }
+    p.k = done;
+    p.bank = i & 1;
     launches.push_back(make_launch(Kind::kBatch2d, 0, BZH_F32, p));
+    done += steps;
   }
   graph_cache().run(s, launches, (a.flags & BZH_FLAG_GRAPH_CACHE) != 0);
 }

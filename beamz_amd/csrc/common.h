@@ -416,44 +416,6 @@ struct DftCapParams {
 };
 void launch_dft_capture(hipStream_t s, const DftCapParams& p);
 
-// One TMxy simulation of a batch on the device: two banks of (Ez, Hx, Hy),
-// uniform decays and H source, an E source array or scalar, CPML memories of
-// both banks (Hx_y, Hy_x, Ez_x, Ez_y), the coefficient table [4][3][2L] and
-// up to four pre-E Ez slab sources.
-struct Sim2dDev {
-  float* ez[2];
-  float* hx[2];
-  float* hy[2];
-  float* psi[2][4];
-  const float* e_src;   // (ny+1, nx+1), or a device scalar when e_src_st == 0
-  const float* e_dec;   // device scalars
-  const float* h_src;
-  const float* h_dec;
-  const float* tab;
-  const float* src_coeff[4];
-  const float* src_wave[4];
-  float inv_dx;
-  int32_t e_src_st;
-  int32_t src_y0[4], src_x0[4], src_sy[4], src_sx[4], src_T[4];
-  int32_t nsrc;
-  int32_t ny, nx, L, metallic;
-};
-
-struct Batch2dParams {
-  const Sim2dDev* sims;
-  const int4* tiles;     // (simulation, item row, item column, 0), queue order
-  int32_t ntiles;
-  int32_t bank;          // bank read by this step
-  const int32_t* step0;  // device scalar: step index of step 0 of this call
-  int32_t k;             // step within this call
-  int32_t tile_rows;     // rows per item (items are 62 columns wide)
-  int32_t workgroups;    // persistent grid size
-  int32_t nsims;         // simulations (the source launch's grid)
-  int32_t max_src_cells; // largest pre-E slab, in cells (0: no sources)
-};
-void launch_batch2d(hipStream_t s, const Batch2dParams& p);
-void launch_batch2d_sources(hipStream_t s, const Batch2dParams& p);
-
 // Several TMxy steps in one launch (tm_steps.hip): float32 fields and CPML
 // memories, scalar H coefficients, one CPML thickness L on every edge (0:
 // none), isotropic metrics.  Bank A (``_in``) is read, bank B written.
@@ -504,6 +466,16 @@ struct TmParams {
   int32_t record_slot;
 };
 void launch_tm(hipStream_t s, const TmParams& p);
+// The same over many simulations: block t runs tile tiles[t] = (simulation,
+// tile row, tile column, 0).
+struct TmBatchParams {
+  const TmSim* sims;
+  const int4* tiles;
+  int32_t ntiles;
+  int32_t rpt, bank, T, k;
+  const int32_t* step0;
+};
+void launch_tm_batch(hipStream_t s, const TmBatchParams& p);
 
 // Reverse-time TMxy step (adjoint.hip).
 struct Adjoint2dParams {

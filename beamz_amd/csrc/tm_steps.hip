@@ -590,6 +590,22 @@ __global__ void __launch_bounds__(64 * NW) tm_steps(TmParams) {
   tm_wave<NW, RPT, kDec, kCpml, true>(S, p->bank, p, rows, T, step, i0, j0);
 }
 
+// Batched simulations: one block per tile of any member, the members'
+// descriptors in device memory.  (One wave per 62-column item, one step per
+// launch and bank B written every step: 121 GCUPS on 64 simulations of 26 M
+// cells; this kernel: see launch_tm_batch.)
+template <int NW, int RPT>
+__global__ void __launch_bounds__(64 * NW) tm_batch(TmBatchParams p) {
+  __shared__ float rows[2][NW][2][64];
+  kptr<int32_t> td = (kptr<int32_t>)(p.tiles + tm_remap(blockIdx.x, gridDim.x));
+  const int sim = td[0], ty = td[1], tx = td[2];
+  const int T = p.T;
+  const int i0 = tx * (64 - 2 * T) - T, j0 = ty * (NW * RPT - 2 * T) - T;
+  const int step = *(kptr<int32_t>)(p.step0) + p.k;
+  tm_wave<NW, RPT, false, true, false>((kptr<TmSim>)(p.sims + sim), p.bank, (kptr<TmParams>)(nullptr),
+                                       rows, T, step, i0, j0);
+}
+
 template <int NW, int RPT>
 void launch_tm_rows(hipStream_t s, const TmParams& p) {
   static_assert(NW * RPT == kTmRows, "tile height");
@@ -614,6 +630,16 @@ void launch_tm(hipStream_t s, const TmParams& p) {
   BZH_REQUIRE(p.ntx * (64 - 2 * p.T) >= p.sim.nx + 1, "2D multi-step tiles do not cover the grid");
   if (p.rpt == 2) launch_tm_rows<16, 2>(s, p);
   else launch_tm_rows<8, 4>(s, p);
+  BZH_HIP(hipGetLastError());
+}
+
+void launch_tm_batch(hipStream_t s, const TmBatchParams& p) {
+  BZH_REQUIRE(p.T >= 1 && p.T <= kTmMaxSteps && (p.rpt == 2 || p.rpt == 4) && p.ntiles >= 1 &&
+                  p.sims != nullptr && p.tiles != nullptr && p.step0 != nullptr,
+              "batched launch is malformed");
+  const dim3 grid(p.ntiles);
+  if (p.rpt == 2) hipLaunchKernelGGL((tm_batch<16, 2>), grid, dim3(64 * 16), 0, s, p);
+  else hipLaunchKernelGGL((tm_batch<8, 4>), grid, dim3(64 * 8), 0, s, p);
   BZH_HIP(hipGetLastError());
 }
 

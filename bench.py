@@ -193,8 +193,8 @@ def run_batched(args):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32",
         "data": "synthetic",
         "config": {"workload": "batched 2D TMxy sweep: 64 simulations, (ny, nx) ~ U{256..1024}^2 at "
-                               "20 nm, 2-4 waveguides, 10-cell CPML, Ez line sources; one persistent "
-                               "launch per step, hipGraph chunks",
+                               "20 nm, 2-4 waveguides, 10-cell CPML, Ez line sources; one launch per "
+                               "several steps, hipGraph chunks",
                    "cells": batch.cells, "simulations": len(batch.progs),
                    "tile_rows": tr, "workgroups": wg},
         "autotune_ms_per_step": {f"{k[0]}x{k[1]}": round(v, 4) for k, v in timings.items()},
@@ -456,12 +456,12 @@ def main():
     ap.add_argument("--per-phase", action="store_true", help="use the per-phase kernels")
     ap.add_argument("--chunk", type=int, default=256)
     ap.add_argument("--tile-rows", type=int, default=0,
-                    help="batched2d: item height (with --workgroups, skips the autotuner)")
-    ap.add_argument("--workgroups", type=int, default=0, help="batched2d: grid size")
+                    help="batched2d: 16 or 32 (with --workgroups, skips the autotuner)")
+    ap.add_argument("--workgroups", type=int, default=0, help="batched2d: unused by the kernel; any non-zero value")
     ap.add_argument("--workload", default="3d", choices=("3d", "waveguide3d", "batched2d", "adjoint2d"),
                     help="3d: the 1024x512x256 Yee+CPML step (default); waveguide3d: the 512x256x128 "
                          "silicon strip; batched2d: the 64-simulation "
-                         "2D sweep in one persistent launch per step; adjoint2d: the 600x600 bend "
+                         "2D sweep, several steps per launch; adjoint2d: the 600x600 bend "
                          "gradient and its finite-difference check")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="run only a 1 GiB device-to-device copy (the byte-counter calibration "

@@ -251,11 +251,10 @@ int32_t bzh_program_noalloc(void* stream, const bzh_buffer* args, int32_t nargs,
 /* ---- batched 2D simulations ------------------------------------------------
  * No counterpart in the reference, which runs one simulation per call (its
  * FFI is vmapped sequentially, cuda/runtime.py:85).  Many independent TMxy
- * (Ez, Hx, Hy) simulations of uneven sizes advance together: each step is
- * one source launch (the pre-E slabs) and one march launch whose waves take
- * the work items (62 columns by tile_rows rows) of every simulation
- * round-robin and march up their rows; a call of nsteps steps is captured
- * once as a hipGraph and replayed.  Two field banks per simulation: bank 0 is
+ * (Ez, Hx, Hy) simulations of uneven sizes advance together: every
+ * simulation is cut into tiles, and one launch advances the tiles of all of
+ * them by up to eight steps; a call of nsteps steps is captured once as a
+ * hipGraph and replayed.  Two field banks per simulation: bank 0 is
  * read by the first step, and after an odd step count the result is in bank
  * 1 (the caller swaps the roles).  All buffers f32. */
 typedef struct bzh_sim2d {
@@ -281,8 +280,8 @@ typedef struct bzh_batch_attrs {
   int32_t abi_version;
   int32_t flags;           /* BZH_FLAG_GRAPH_CACHE */
   int32_t nsteps;
-  int32_t tile_rows;       /* rows per work item (62 columns wide): 8, 16, 32 or 64 */
-  int32_t workgroups;      /* persistent grid size; 0 picks 4 per compute unit */
+  int32_t tile_rows;       /* 8 or 16: two rows per lane; 32 or 64: four */
+  int32_t workgroups;      /* unused (every tile is its own workgroup) */
 } bzh_batch_attrs;
 
 /* current_step: s32 device scalar, the step index of the first step. */
