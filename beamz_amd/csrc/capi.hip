@@ -870,6 +870,18 @@ bool fused_banded() {
   return !(env && std::string(env) == "xcd");
 }
 
+// Tiles per band of a box of ``tiles`` tiles, 0 for the contiguous-range
+// order.  Bands give each XCD ceil(tiles / 8) tile columns: with few tiles
+// some XCDs get twice the work of others (24 tile columns in three boxes of
+// 64x96x128: 57 against 54 us per step), so boxes below 64 tiles, where the
+// fullest XCD can hold more than 9/8 of its share, are dealt evenly
+// block by block instead.  ``fixed``: see pair_kz.
+constexpr int64_t kBandTiles = 64;
+int band_tiles(int64_t tiles, bool fixed) {
+  if (!fused_banded() || (!fixed && tiles < kBandTiles)) return 0;
+  return static_cast<int>((tiles + 7) / 8);
+}
+
 FusedSplit fused_split(const Grid& g, int L) {
   const int TY = fused_rows();
   const int Tx = (g.nx + 1 + 61) / 62, Ty = (g.ny + 1 + TY - 1) / TY, planes = g.nz + 1;
@@ -918,16 +930,20 @@ struct PairSplit {
 // Chunk depth of a pair launch.  A block marches kz owned planes plus three to
 // four of start-up and lag, one 16-wave block per CU, so a launch of B blocks
 // takes about max(B, 256) (kz + 3): below 256 blocks shorter chunks are free
-// parallelism, above it they only add start-up planes.  The chunk count that
+// parallelism, above it they only add start-up planes.  Without a core box
+// all blocks take equally long and rounds of 256 count whole (at 64x96x128,
+// 264 blocks of 6 planes take 54 us per step, 240 of 7 planes 50); with one,
+// its shorter blocks fill the last round (at 97x150x263, 300 blocks of 20
+// planes take 105 us, 240 of 25 planes 112).  The chunk count that
 // minimizes this, with chunks of 3 to 48 planes (2-plane chunks measured 25 %
 // slower than 3 at 40x60x80), per step with a plane source and a flux plane:
-// 64x96x128 153 -> 49 us, 97x150x263 179 -> 111 us, 40x60x80 147 -> 35 us,
+// 64x96x128 153 -> 47 us, 97x150x263 179 -> 111 us, 40x60x80 147 -> 35 us,
 // 128x256x512 253 -> 249 us, against 48 planes at every size.
 // ``fixed``: stochastic bfloat16 rounding draws by block, so its schedule
 // (and with it every rounded bit) stays that of 48-plane chunks.
 constexpr int kPairBlocks = 256;
 constexpr int kPairKzMin = 3, kPairKzMax = 48;
-int pair_kz(int64_t tiles, int planes, bool fixed) {
+int pair_kz(int64_t tiles, int planes, bool core, bool fixed) {
   if (const char* env = std::getenv("BZH_PAIR_KZ")) return std::max(1, std::atoi(env));
   if (fixed || tiles <= 0) return kPairKzMax;
   int best = 0;
@@ -936,7 +952,8 @@ int pair_kz(int64_t tiles, int planes, bool fixed) {
     const int kz = (planes + n - 1) / n;
     if (best > 0 && kz < kPairKzMin) break;
     const int64_t blocks = tiles * ((planes + kz - 1) / kz);
-    const int64_t cost = std::max<int64_t>(blocks, kPairBlocks) * (kz + 3);
+    const int64_t rounds = (blocks + kPairBlocks - 1) / kPairBlocks;
+    const int64_t cost = (core ? std::max<int64_t>(blocks, kPairBlocks) : rounds * kPairBlocks) * (kz + 3);
     if (best == 0 || cost < best_cost) {
       best = kz;
       best_cost = cost;
@@ -947,7 +964,7 @@ int pair_kz(int64_t tiles, int planes, bool fixed) {
 
 // Finish a box: z chunking over [z0, zsplit) and [zhi, z1) with chunks of at
 // most kz planes, bands and block count; returns false for an empty box.
-bool finish_box(PairBox& b, int kz, bool even) {
+bool finish_box(PairBox& b, int kz, bool even, bool fixed) {
   const int64_t tiles = static_cast<int64_t>(b.ntx) * b.nty;
   auto chunks = [&](int n) {
     if (n <= 0) return std::pair<int, int>(0, kz);
@@ -960,7 +977,7 @@ bool finish_box(PairBox& b, int kz, bool even) {
   b.nzc_lo = b.zsplit > b.z0 ? (b.zsplit - b.z0 + b.kz - 1) / b.kz : 0;
   b.nzc = b.nzc_lo + (b.z1 > b.zhi ? (b.z1 - b.zhi + b.kz - 1) / b.kz : 0);
   if (tiles == 0 || b.nzc == 0) return false;
-  b.band = fused_banded() ? static_cast<int>((tiles + 7) / 8) : 0;
+  b.band = band_tiles(tiles, fixed);
   const int64_t n = (b.band > 0 ? 8 * int64_t{b.band} : tiles) * b.nzc;
   b.nblk = static_cast<int32_t>((n + 7) / 8 * 8);
   return true;
@@ -973,7 +990,6 @@ PairSplit pair_split(const Grid& g, int L, bool fixed_kz) {
   int tx0 = (M + 2 + W - 1) / W;                           // W tx0 - 2 >= M
   int tx1 = g.nx - M - 2 >= 0 ? std::min((g.nx - M - 2) / W, Tx) : 0;  // W tx1 <= nx - M - 2
   if (tx1 <= tx0) tx0 = tx1 = 0;
-  const int kz = pair_kz(int64_t{Tx} * Ty, planes, fixed_kz);
   // core rows: 13 by - 2 >= M and 13 by + 13 <= ny - L - 1
   const int cy0 = (M + 2 + TY - 1) / TY;
   const int cy1 = g.ny - L - 1 - TY >= 0 ? (g.ny - L - 1 - TY) / TY + 1 : 0;
@@ -981,6 +997,7 @@ PairSplit pair_split(const Grid& g, int L, bool fixed_kz) {
   const int cz0 = M + 4, cz1 = g.nz - M - 3;
   const char* env = std::getenv("BZH_PAIR_CORE");
   const bool core = !(env && std::string(env) == "0") && tx1 > tx0 && cy1 > cy0 && cz1 > cz0;
+  const int kz = pair_kz(int64_t{Tx} * Ty, planes, core, fixed_kz);
   PairSplit sp;
   auto box = [&](int bx0, int ntx, int tsplit, int tskip, int by0, int nty, int tysplit, int tyskip,
                  int z0, int zsplit, int zhi, int z1, int xedge) {
@@ -1002,22 +1019,22 @@ PairSplit pair_split(const Grid& g, int L, bool fixed_kz) {
   };
   // the x-edge tiles (slower: first, so that they do not form the tail)
   PairBox e = box(0, tx0 + (Tx - tx1), tx0, tx1 - tx0, 0, Ty, Ty, 0, 0, planes, planes, planes, 1);
-  if (finish_box(e, kz, false)) sp.shell[sp.nshell++] = e;
+  if (finish_box(e, kz, false, fixed_kz)) sp.shell[sp.nshell++] = e;
   if (!core) {
     PairBox in = box(tx0, tx1 - tx0, tx1 - tx0, 0, 0, Ty, Ty, 0, 0, planes, planes, planes, 0);
-    if (finish_box(in, kz, false)) sp.shell[sp.nshell++] = in;
+    if (finish_box(in, kz, false, fixed_kz)) sp.shell[sp.nshell++] = in;
     return sp;
   }
   // x-interior tiles outside the core rows, every plane
   PairBox out = box(tx0, tx1 - tx0, tx1 - tx0, 0, 0, Ty - (cy1 - cy0), cy0, cy1 - cy0, 0, planes,
                     planes, planes, 0);
-  if (finish_box(out, kz, false)) sp.shell[sp.nshell++] = out;
+  if (finish_box(out, kz, false, fixed_kz)) sp.shell[sp.nshell++] = out;
   // x-interior core-row tiles on the planes outside the core range
   PairBox rim = box(tx0, tx1 - tx0, tx1 - tx0, 0, cy0, cy1 - cy0, cy1 - cy0, 0, 0, cz0, cz1, planes, 0);
-  if (finish_box(rim, kz, false)) sp.shell[sp.nshell++] = rim;
+  if (finish_box(rim, kz, false, fixed_kz)) sp.shell[sp.nshell++] = rim;
   // the core, in chunks of equal length
   sp.core = box(tx0, tx1 - tx0, tx1 - tx0, 0, cy0, cy1 - cy0, cy1 - cy0, 0, cz0, cz1, cz1, cz1, 2);
-  sp.has_core = finish_box(sp.core, kz, true);
+  sp.has_core = finish_box(sp.core, kz, true, fixed_kz);
   if (sp.has_core && !(env && std::string(env) == "split")) {
     sp.shell[sp.nshell++] = sp.core;
     sp.has_core = false;
@@ -1795,7 +1812,7 @@ bool run_program(hipStream_t s, ProgramIn& in) {
     fp.box_nty = b.nty;
     fp.box_kz = b.kz;
     fp.box_nzc = b.nzc;
-    fp.box_band = fused_banded() ? (b.ntx * b.nty + 7) / 8 : 0;
+    fp.box_band = band_tiles(int64_t{b.ntx} * b.nty, fp.bf16_sr != 0);
   };
 
   std::vector<Launch> launches;
