@@ -138,6 +138,7 @@ struct PhaseParams {
   float inv_dx;
   int32_t metallic;     // bit mask of PEC faces
   int32_t nz, ny, nx;   // material grid
+  int32_t run;          // blocks per run of the 3D launches (set there)
   int32_t nterms;       // 0 or 6 (3D) / 0 or 2 (TMxy)
   int32_t uniform_l;    // uniform CPML thickness (0 -> read metadata)
   const int32_t* meta;  // term metadata s32[nterms, 5] (device)

@@ -1,0 +1,43 @@
+"""The 3D per-phase kernels against the FP64 oracle, at sizes around the ends of
+a wave's 64 cells and of a 4-row block, where waves change between the plain,
+x-edge and general bodies, with scalar and per-cell coefficients, CPML on all
+and on some faces, metal faces, and grids too thin for any plain wave.
+
+Tolerance: the FP32-against-FP64 bounds of the parity tests (``_close``).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import fdtd64 as o
+from tests.test_gpu_parity import _compare_state, _require_gpu, _setup
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lossy", [False, True], ids=["uniform", "lossy"])
+@pytest.mark.parametrize("grid,cpml,faces,metal", [
+    ((1, 1, 1), None, None, ("left", "top")),
+    ((3, 5, 63), None, None, None),
+    ((9, 8, 64), 2, None, None),
+    ((10, 13, 65), 3, ("left", "right"), ("bottom", "back")),
+    ((12, 7, 128), 3, None, ("front",)),
+    ((9, 12, 129), 1, ("front", "back", "top"), None),
+    ((11, 18, 200), 4, None, None),
+    ((30, 3, 2), None, None, ("front", "back", "bottom", "top", "left", "right"))])
+def test_phase_kernels_parity(grid, cpml, faces, metal, lossy):
+    _require_gpu()
+    print(f"case phase3d grid={grid} cpml={cpml} faces={faces} metal={metal} lossy={lossy}", flush=True)
+    sigma = None
+    if lossy:
+        sigma = np.random.default_rng(7).uniform(0.0, 2e4, grid)
+    steps = 12
+    sim, prog, state, prob, ost = _setup(grid, seed=57, steps=steps, cpml_cells=cpml, faces=faces,
+                                         metallic=metal, fused=False, sigma=sigma)
+    state = sim.advance(state, steps)
+    torch.cuda.synchronize()
+    o.run(prob, ost, steps)
+    _compare_state(prog, state, prob, ost)
