@@ -1817,8 +1817,18 @@ bool run_program(hipStream_t s, ProgramIn& in) {
 
   std::vector<Launch> launches;
   launches.reserve(static_cast<size_t>(in.nsteps) * 8);
-  // the DFT of step k, read from ``bank`` (buffered: stage, and fold the ring
-  // every ``slots`` steps and at the end of the call)
+  // buffered DFT: fold the ring after step k when its last slot is filled, and
+  // at the end of the call
+  auto add_flush = [&](DftParams dp, int k) {
+    if ((k + 1) % slots != 0 && k != in.nsteps - 1) return;
+    dp.mode = 2;
+    dp.slots = slots;
+    dp.stage = stage;
+    dp.nk = (k % slots) + 1;
+    dp.k0 = k + 1 - dp.nk;
+    launches.push_back(make_launch(Kind::kDft, 0, g.dtype, dp));
+  };
+  // the DFT of step k, read from ``bank``
   auto add_dft = [&](int k, const bzh_buffer* const* bank) {
     DftParams dp = make_dft(in.mon, bank, g, in.dt, in.monitor_count);
     dp.k = k;
@@ -1827,15 +1837,32 @@ bool run_program(hipStream_t s, ProgramIn& in) {
       dp.slots = slots;
       dp.stage = stage;
       launches.push_back(make_launch(Kind::kDft, 0, g.dtype, dp));
-      if ((k + 1) % slots == 0 || k == in.nsteps - 1) {
-        dp.mode = 2;
-        dp.nk = (k % slots) + 1;
-        dp.k0 = k + 1 - dp.nk;
-        launches.push_back(make_launch(Kind::kDft, 0, g.dtype, dp));
-      }
+      add_flush(dp, k);
     } else {
       launches.push_back(make_launch(Kind::kDft, 0, g.dtype, dp));
     }
+  };
+  // the DFT of a pair's steps k (from ``mid`` or the capture) and k + 1 (from
+  // ``last``), both staged by one launch
+  auto add_dft_pair = [&](int k, const bzh_buffer* const* mid, const bzh_buffer* const* last) {
+    DftParams dp = make_dft(in.mon, last, g, in.dt, in.monitor_count);
+    dp.k = k;
+    dp.mode = 1;
+    dp.slots = slots;
+    dp.stage = stage;
+    dp.pair = 1;
+    for (int c = 0; c < 6; ++c) dp.field2[c] = dp.field[c];
+    if (cap.ok) {
+      dp.cap = pws.cap;
+      dp.capbox = pws.capbox;
+    } else {
+      const DftParams first = make_dft(in.mon, mid, g, in.dt, in.monitor_count);
+      for (int c = 0; c < 6; ++c) dp.field[c] = first.field[c];
+    }
+    launches.push_back(make_launch(Kind::kDft, 0, g.dtype, dp));
+    DftParams fp = make_dft(in.mon, last, g, in.dt, in.monitor_count);
+    fp.k = k + 1;
+    add_flush(fp, k + 1);
   };
   // the DFT of the pair's first step, from the capture
   auto add_dft_cap = [&](int k) {
@@ -1925,16 +1952,19 @@ bool run_program(hipStream_t s, ProgramIn& in) {
         pc.core = 1;
         launches.push_back(make_launch(Kind::kPair, 0, g.dtype, pc));
       }
-      if (in.has_monitors && cap.ok) {
+      // (a ring that ends between the two steps, or none, keeps two launches)
+      const bool dft_pair = in.has_monitors && slots > 1 && (k + 1) % slots != 0;
+      if (in.has_monitors && !dft_pair && cap.ok) {
         add_dft_cap(k);
-      } else if (in.has_monitors) {
+      } else if (in.has_monitors && !dft_pair) {
         add_dft(k, cbank);
       }
       for (int c = 0; c < 3 && 6 + c < in.ngroups; ++c)
         add_source_launches(launches, in.groups[6 + c], 2, c, nxt, g, in.metallic, step0, k + 1);
       // (the second step is sampled from the fields: capturing it too costs
       // the kernel more stores than the strided gather costs)
-      if (in.has_monitors) add_dft(k + 1, nxt);
+      if (dft_pair) add_dft_pair(k, cbank, nxt);
+      else if (in.has_monitors) add_dft(k + 1, nxt);
       --pairs_left;
       cur_b = two_banks ? !cur_b : cur_b;
       k += 2;

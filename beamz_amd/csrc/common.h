@@ -396,6 +396,9 @@ struct DftParams {
   const float* cap;
   const int32_t* capbox;
   int32_t fdims[6][3];   // component shapes (z, y, x), for the capture index
+  // mode 1: stage step k + 1 too, from these fields
+  int32_t pair;
+  const void* field2[6];
 };
 constexpr int kDftMaxSlots = 32;
 void launch_dft(hipStream_t s, const DftParams& p);

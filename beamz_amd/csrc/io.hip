@@ -50,31 +50,44 @@ constexpr int kMaxFreq = 256;
 // Weighted gather of one monitor sample (observe.py:360-370, 529-585),
 // from the field or, when ``p.cap`` is set, from the capture of the
 // monitored cells (the corner's cell mapped into its component's box).
+//
+// Four corners at a time: their indices and weights, then their cells, are
+// loaded before the first is summed (one corner after another cost three
+// dependent round trips each).  Corners outside the component add nothing, and
+// are read at element 0 instead.
 template <typename T>
-__device__ __forceinline__ float gather(const DftParams& p, int m, int c, int pt) {
-  const T* fld = static_cast<const T*>(p.field[c]);
+__device__ __forceinline__ float gather(const DftParams& p, const T* fld, const float* cap, int m,
+                                        int c, int pt) {
   const int64_t base = ((static_cast<int64_t>(m) * 6 + c) * p.Pmax + pt) * p.K;
+  const int32_t* t = p.capbox + (m * 6 + c) * 8;
+  const int sy = p.fdims[c][1], sx = p.fdims[c][2];
   float v = 0.0f;
-  if (p.cap != nullptr) {
-    const int32_t* t = p.capbox + (m * 6 + c) * 8;
-    const int z0 = t[0], z1 = t[1], y0 = t[2], y1 = t[3], x0 = t[4], x1 = t[5];
-    const int sy = p.fdims[c][1], sx = p.fdims[c][2];
-    const int nzb = z1 - z0 + 1, nyb = y1 - y0 + 1;
-    for (int q = 0; q < p.K; ++q) {
-      const int idx = p.indices[base + q];
-      const float w = p.weights[base + q];
-      if (w == 0.0f || idx < 0 || idx >= p.fsize[c]) continue;
-      const int z = idx / (sy * sx), r = idx - z * (sy * sx);
-      const int y = r / sx, x = r - y * sx;
-      if (z < z0 || z > z1 || y < y0 || y > y1 || x < x0 || x > x1) continue;
-      v += w * p.cap[t[6] + ((x - x0) * nyb + (y - y0)) * nzb + (z - z0)];
+  for (int q0 = 0; q0 < p.K; q0 += 4) {
+    int idx[4];
+    float w[4], x[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int q = min(q0 + e, p.K - 1);
+      idx[e] = p.indices[base + q];
+      w[e] = q0 + e < p.K ? p.weights[base + q] : 0.0f;
     }
-    return v;
-  }
-  for (int q = 0; q < p.K; ++q) {
-    const int idx = p.indices[base + q];
-    const float w = p.weights[base + q];
-    if (w != 0.0f && idx >= 0 && idx < p.fsize[c]) v += w * load_f(fld, idx);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (idx[e] < 0 || idx[e] >= p.fsize[c]) w[e] = 0.0f;
+      int cell = w[e] != 0.0f ? idx[e] : 0;
+      if (cap != nullptr) {
+        const int nzb = t[1] - t[0] + 1, nyb = t[3] - t[2] + 1;
+        const int cz = cell / (sy * sx), r = cell - cz * (sy * sx);
+        const int cy = r / sx, cx = r - cy * sx;
+        if (cz < t[0] || cz > t[1] || cy < t[2] || cy > t[3] || cx < t[4] || cx > t[5]) w[e] = 0.0f;
+        cell = w[e] != 0.0f ? t[6] + ((cx - t[4]) * nyb + (cy - t[2])) * nzb + (cz - t[0]) : 0;
+        x[e] = cap[cell];
+      } else {
+        x[e] = load_f(fld, cell);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v = w[e] != 0.0f ? v + w[e] * x[e] : v;
   }
   return v;
 }
@@ -112,18 +125,26 @@ __device__ __forceinline__ bool dft_gate(const DftParams& p, int m, int k, doubl
   return true;
 }
 
-// Buffered path, step k: stage the gathered sample (f32) in ring slot k % slots.
+// Buffered path, step k: stage the gathered sample (f32) in ring slot k % slots;
+// with p.pair also step k + 1's, from field2 (blockIdx.y 1).  A strided plane
+// is bound by the lines of its cells, a small one by the launch: three
+// 128 x 256 planes normal to x take 26 us for both steps (two launches: 34),
+// two 64 x 96 ones 5.5 us (11).
 template <typename T>
 __global__ void __launch_bounds__(kDftBlock) dft_stage_kernel(DftParams p) {
   const int m = blockIdx.z / 6;
   const int c = blockIdx.z % 6;
+  const bool second = blockIdx.y != 0;
+  const int k = p.k + blockIdx.y;
   const int P = p.counts[m * 5 + 1];
   double t, window, scale;
-  if (!dft_gate(p, m, p.k, t, window, scale)) return;
+  if (!dft_gate(p, m, k, t, window, scale)) return;
   const int pt = blockIdx.x * kDftBlock + threadIdx.x;
-  if (p.masks[m * 6 + c] == 0.0f || pt >= P || pt >= p.Pmax || p.field[c] == nullptr) return;
-  const int64_t slot = p.k % p.slots;
-  p.stage[((slot * p.M + m) * 6 + c) * p.Pmax + pt] = gather<T>(p, m, c, pt);
+  const T* fld = static_cast<const T*>(second ? p.field2[c] : p.field[c]);
+  if (p.masks[m * 6 + c] == 0.0f || pt >= P || pt >= p.Pmax || fld == nullptr) return;
+  const int64_t slot = k % p.slots;
+  p.stage[((slot * p.M + m) * 6 + c) * p.Pmax + pt] =
+      gather<T>(p, fld, second ? nullptr : p.cap, m, c, pt);
 }
 
 // Fold steps k0 .. k0+nk-1 into the accumulators of frequencies f0 .. f0+kFt-1
@@ -363,7 +384,7 @@ __global__ void __launch_bounds__(kDftBlock) dft_kernel(DftParams p) {
   const float cmask = p.masks[m * 6 + c];
   const int pt = blockIdx.x * kDftBlock + threadIdx.x;
   if (cmask == 0.0f || pt >= P || pt >= p.Pmax || p.field[c] == nullptr) return;
-  const float v = gather<T>(p, m, c, pt);
+  const float v = gather<T>(p, static_cast<const T*>(p.field[c]), p.cap, m, c, pt);
   const double dv = static_cast<double>(v) * p.inv_scale[c] * cmask * scale;
   A* re = static_cast<A*>(p.re);
   A* im = static_cast<A*>(p.im);
@@ -381,6 +402,7 @@ void dft_dispatch(hipStream_t s, const DftParams& p) {
   dim3 block(kDftBlock, 1, 1);
   dim3 grid((p.Pmax + kDftBlock - 1) / kDftBlock, 1, p.M * 6);
   if (p.mode == 1) {
+    grid.y = p.pair != 0 ? 2 : 1;
     hipLaunchKernelGGL((dft_stage_kernel<T>), grid, block, 0, s, p);
   } else if (p.mode == 2) {
     grid.y = (p.Fmax + kFt - 1) / kFt;
@@ -471,7 +493,9 @@ void launch_dft(hipStream_t s, const DftParams& p) {
   BZH_REQUIRE(p.Fmax <= kMaxFreq, "DFT monitors support at most 256 frequencies");
   if (p.mode != 0) {
     BZH_REQUIRE(p.stage != nullptr && p.slots >= 1 && p.slots <= kDftMaxSlots,
-                "buffered DFT needs a staging ring of 1..16 slots");
+                "buffered DFT needs a staging ring of 1..32 slots");
+    BZH_REQUIRE(p.pair == 0 || (p.mode == 1 && (p.k + 1) % p.slots != 0),
+                "a pair of DFT samples needs two slots of one ring round");
     BZH_REQUIRE(p.mode != 2 || (p.nk >= 1 && p.nk <= p.slots), "DFT flush range exceeds the ring");
   }
   switch (p.dtype) {
