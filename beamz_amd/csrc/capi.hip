@@ -637,7 +637,7 @@ void add_source_launches(std::vector<Launch>& out, const SourceGroupIn& grp, int
   }
 }
 
-// Fold a timed source group into a 2D phase launch (PhaseParams::psrc): the
+// Fold a timed source group into a phase launch (PhaseParams::psrc): the
 // checks of add_source_launches, then the group's slabs, summed per cell in
 // declaration order inside the kernel.
 void fold_phase_sources(PhaseParams& p, const SourceGroupIn& grp, int comp_in_phase, int comp,
@@ -647,7 +647,8 @@ void fold_phase_sources(PhaseParams& p, const SourceGroupIn& grp, int comp_in_ph
   if (c.data == nullptr || c.rank < 1 || c.dims[0] == 0) return;
   const int n = static_cast<int>(c.dims[0]);
   const bzh_buffer& field = *bank[comp];
-  BZH_REQUIRE(field.data != nullptr && field.rank == 2, "source targets an absent field component");
+  BZH_REQUIRE(field.data != nullptr && field.rank == (g.is3d ? 3 : 2),
+              "source targets an absent field component");
   BZH_REQUIRE(c.element_type == BZH_F32 && grp.waves->element_type == BZH_F32 &&
                   grp.starts->element_type == BZH_S32,
               "source groups are f32 coefficients, f32 waveforms and s32 starts");
@@ -656,8 +657,8 @@ void fold_phase_sources(PhaseParams& p, const SourceGroupIn& grp, int comp_in_ph
   BZH_REQUIRE(grp.starts->rank == 2 && grp.starts->dims[0] == n && grp.starts->dims[1] == 3,
               "source starts must be s32[n, 3]");
   BZH_REQUIRE(c.rank == 4, "source coefficients must be [n, sz, sy, sx]");
-  BZH_REQUIRE(p.npsrc < kMaxPhaseSrc, "too many folded source groups");
-  PhaseSrc& q = p.psrc[p.npsrc++];
+  PhaseSrc& q = p.psrc[comp_in_phase];
+  ++p.npsrc;
   q.coeff = static_cast<const float*>(c.data);
   q.wave = static_cast<const float*>(grp.waves->data);
   q.starts = static_cast<const int32_t*>(grp.starts->data);
@@ -666,9 +667,9 @@ void fold_phase_sources(PhaseParams& p, const SourceGroupIn& grp, int comp_in_ph
   q.sy = static_cast<int>(c.dims[2]);
   q.sx = static_cast<int>(c.dims[3]);
   q.T = static_cast<int>(grp.waves->dims[1]);
-  q.comp = comp_in_phase;
-  q.fy = static_cast<int>(field.dims[0]);
-  q.fx = static_cast<int>(field.dims[1]);
+  q.fz = g.is3d ? static_cast<int>(field.dims[0]) : 1;
+  q.fy = static_cast<int>(field.dims[field.rank - 2]);
+  q.fx = static_cast<int>(field.dims[field.rank - 1]);
   mask_ends(comp, metallic, g.is3d, q.mlo, q.mhi);
   p.step0 = step0;
   p.k = k;
@@ -1893,13 +1894,15 @@ bool run_program(hipStream_t s, ProgramIn& in) {
   }
 
   const Kind pk = g.is3d ? Kind::kPhase3d : Kind::kPhaseTm;
-  // 2D float32 programs fold their timed source slabs into the phase launches
-  // (three launches per step instead of five: H, E, the DFT sample); the
-  // groups that do not fit keep their source launches
-  bool fold_tm = !g.is3d && g.dtype == BZH_F32 && step0 != nullptr;
-  for (int c = 0; c < 3 && fold_tm; ++c) {
-    if (3 + c < in.ngroups && group_slabs(in.groups[3 + c]) > 0 && c == 2) fold_tm = false;  // (no Hz in TMxy)
-    if (6 + c < in.ngroups && group_slabs(in.groups[6 + c]) > 0 && c < 2) fold_tm = false;  // (no Ex, Ey)
+  // float32 programs fold their timed source slabs into the phase launches: a
+  // launch of its own costs 5 us, as much as a small phase (2D: three launches
+  // per step instead of five, H, E and the DFT sample; 64x112x160 with
+  // electric and magnetic sheets: 51 -> 48.5 us per step); the groups that do
+  // not fit keep their source launches
+  bool fold = g.dtype == BZH_F32 && step0 != nullptr;
+  for (int c = 0; c < 3 && fold && !g.is3d; ++c) {
+    if (3 + c < in.ngroups && group_slabs(in.groups[3 + c]) > 0 && c == 2) fold = false;  // (no Hz in TMxy)
+    if (6 + c < in.ngroups && group_slabs(in.groups[6 + c]) > 0 && c < 2) fold = false;  // (no Ex, Ey)
   }
   bool cur_b = false;  // the current fields live in bank B
   int pairs_left = npairs;
@@ -1995,21 +1998,20 @@ bool run_program(hipStream_t s, ProgramIn& in) {
       }
       PhaseParams hp = make_phase(h, BZH_PHASE_H, g, in.dt, in.resolution, in.metallic, in.uniform_l);
       PhaseParams ep = make_phase(e, BZH_PHASE_E, g, in.dt, in.resolution, in.metallic, in.uniform_l);
-      if (fold_tm) {
-        // 2D, float32: the H-timed slabs (Hx, Hy) and the E-timed ones (Ez)
-        // run inside the phase launches
-        for (int c = 0; c < 2 && 3 + c < in.ngroups; ++c)
+      if (fold) {
+        // the H-timed slabs and the E-timed ones run inside the phase launches
+        for (int c = 0; c < 3 && 3 + c < in.ngroups; ++c)
           fold_phase_sources(hp, in.groups[3 + c], c, kHx + c, nxt, g, in.metallic, step0, k);
-        if (8 < in.ngroups)
-          fold_phase_sources(ep, in.groups[8], 2, kEz, nxt, g, in.metallic, step0, k);
+        for (int c = 0; c < 3 && 6 + c < in.ngroups; ++c)
+          fold_phase_sources(ep, in.groups[6 + c], c, kEx + c, nxt, g, in.metallic, step0, k);
       }
       launches.push_back(make_launch(pk, BZH_PHASE_H, g.dtype, hp));
-      if (!fold_tm)
+      if (!fold)
         for (int c = 0; c < 3 && 3 + c < in.ngroups; ++c)
           add_source_launches(launches, in.groups[3 + c], 1, c, nxt, g, in.metallic, step0, k);
       launches.push_back(make_launch(pk, BZH_PHASE_E, g.dtype, ep));
     }
-    if (!fold_tm)
+    if (fused || !fold)
       for (int c = 0; c < 3 && 6 + c < in.ngroups; ++c)
         add_source_launches(launches, in.groups[6 + c], 2, c, nxt, g, in.metallic, step0, k);
     if (in.has_monitors) add_dft(k, nxt);

@@ -111,11 +111,9 @@ struct PhaseSrc {
   const float* wave;       // [n, T]
   const int32_t* starts;   // [n, 3] (z, y, x)
   int32_t n, sz, sy, sx, T;
-  int32_t comp;
-  int32_t fy, fx;          // the target's shape (rows, columns)
+  int32_t fz, fy, fx;      // the target's shape (planes, rows, columns)
   int32_t mlo[3], mhi[3];  // PEC-constrained ends (z, y, x)
 };
-constexpr int kMaxPhaseSrc = 2;
 
 struct PhaseParams {
   const void* tin[3];   // targets read
@@ -143,9 +141,9 @@ struct PhaseParams {
   int32_t uniform_l;    // uniform CPML thickness (0 -> read metadata)
   const int32_t* meta;  // term metadata s32[nterms, 5] (device)
   DevTerm term[6];
-  // timed source slabs of this step folded into the 2D kernels (npsrc 0: the
+  // timed source slabs of this step folded into the kernels (npsrc 0: the
   // source launches apply them); the waveform index is *step0 + k
-  PhaseSrc psrc[kMaxPhaseSrc];
+  PhaseSrc psrc[3];      // by target component; n 0: none
   int32_t npsrc;
   const int32_t* step0;
   int32_t k;

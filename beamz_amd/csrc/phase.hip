@@ -84,6 +84,58 @@ __device__ __forceinline__ float scf_at(const PhaseParams& p, int c, int o) {
   return coef(p.scf[c], p.scf_st[c], p.scf_s[c], o);
 }
 
+// What folded source group ``s`` adds to its target's cell (k, j, i), the
+// slabs in declaration order after v (as successive source launches add them,
+// to rounding); float32 fields only.
+__device__ __forceinline__ float group_add(const PhaseParams& p, const PhaseSrc& s, int k, int j,
+                                           int i, float v) {
+  if ((s.mlo[0] && k == 0) || (s.mhi[0] && k == s.fz - 1) || (s.mlo[1] && j == 0) ||
+      (s.mhi[1] && j == s.fy - 1) || (s.mlo[2] && i == 0) || (s.mhi[2] && i == s.fx - 1))
+    return v;
+  int widx = *p.step0 + p.k;
+  widx = widx < 0 ? 0 : (widx > s.T - 1 ? s.T - 1 : widx);
+  for (int q = 0; q < s.n; ++q) {
+    const int cz = k - s.starts[q * 3 + 0], cy = j - s.starts[q * 3 + 1];
+    const int cx = i - s.starts[q * 3 + 2];
+    if (cz < 0 || cz >= s.sz || cy < 0 || cy >= s.sy || cx < 0 || cx >= s.sx) continue;
+    const int64_t c = ((static_cast<int64_t>(q) * s.sz + cz) * s.sy + cy) * s.sx + cx;
+    v = v + s.coeff[c] * s.wave[static_cast<int64_t>(q) * s.T + widx];
+  }
+  return v;
+}
+// the groups of a 3D phase's three targets.  Few waves meet a source, so the
+// parameters are re-read from the argument block through a pointer the
+// compiler cannot see into: read as ordinary arguments they were all loaded
+// at the kernel's start and spilled (4591 against 3930 us per 64 lossy steps
+// at 72x120x200).
+__device__ __forceinline__ void sources_3d(int k, int j, int i, float& x, float& y, float& z) {
+  using KP = __attribute__((address_space(4))) const PhaseParams;
+  KP* a = (KP*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  for (int c = 0; c < 3; ++c) {
+    const auto& s = a->psrc[c];
+    if (s.n == 0) continue;
+    float add = 0.0f;
+    for (int q = 0; q < s.n; ++q) {
+      const int cz = k - s.starts[q * 3 + 0], cy = j - s.starts[q * 3 + 1];
+      if (cz < 0 || cz >= s.sz || cy < 0 || cy >= s.sy) continue;
+      if ((s.mlo[0] && k == 0) || (s.mhi[0] && k == s.fz - 1) || (s.mlo[1] && j == 0) ||
+          (s.mhi[1] && j == s.fy - 1))
+        continue;
+      const int cx = i - s.starts[q * 3 + 2];
+      const bool open = !((s.mlo[2] && i == 0) || (s.mhi[2] && i == s.fx - 1));
+      int widx = *a->step0 + a->k;
+      widx = widx < 0 ? 0 : (widx > s.T - 1 ? s.T - 1 : widx);
+      const float wv = s.wave[static_cast<int64_t>(q) * s.T + widx];
+      if (open && cx >= 0 && cx < s.sx)
+        add += s.coeff[((static_cast<int64_t>(q) * s.sz + cz) * s.sy + cy) * s.sx + cx] * wv;
+    }
+    x += c == 0 ? add : 0.0f;
+    y += c == 1 ? add : 0.0f;
+    z += c == 2 ? add : 0.0f;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // 3D phases
 //
@@ -230,6 +282,7 @@ __device__ __forceinline__ void h_cell(const PhaseParams& p, int i, int j, int k
   if (kX && (((m & kLeft) && i == 0) || ((m & kRight) && i == nx))) hx = 0.0f;
   if (kYZ && (((m & kBottom) && j == 0) || ((m & kTop) && j == ny))) hy = 0.0f;
   if (kYZ && (((m & kFront) && k == 0) || ((m & kBack) && k == nz))) hz = 0.0f;
+  if (p.npsrc > 0) sources_3d(k, j, i, hx, hy, hz);
   if (vk && vj && vY) stb<T>(p.tout[0], ox * sz, hx);
   if (vk && vX) stb<T>(p.tout[1], oy * sz, hy);
   if (vj && vX) stb<T>(p.tout[2], oz * sz, hz);
@@ -296,6 +349,7 @@ __device__ __forceinline__ void e_cell(const PhaseParams& p, int i, int j, int k
   if (zf || yf) ex = 0.0f;
   if (zf || xf) ey = 0.0f;
   if (yf || xf) ez = 0.0f;
+  if (p.npsrc > 0) sources_3d(k, j, i, ex, ey, ez);
   if (vX) stb<T>(p.tout[0], ox * sz, ex);
   if (vj && vY) stb<T>(p.tout[1], oy * sz, ey);
   if (vk && vY) stb<T>(p.tout[2], oz * sz, ez);
@@ -335,28 +389,6 @@ phase_3d(PhaseParams p) {
 // 2D TMxy (Ez, Hx, Hy) on (ny, nx): kernels.py:731-811, 1217-1290
 // ---------------------------------------------------------------------------
 
-// The folded timed source slabs of target ``comp`` at cell (j, i), added to
-// the updated value v in declaration order (as successive source launches
-// add them, to rounding); float32 fields only.
-__device__ __forceinline__ float tm_sources(const PhaseParams& p, int comp, int j, int i, float v) {
-  for (int g = 0; g < p.npsrc; ++g) {
-    const PhaseSrc& s = p.psrc[g];
-    if (s.comp != comp) continue;
-    if ((s.mlo[1] && j == 0) || (s.mhi[1] && j == s.fy - 1) || (s.mlo[2] && i == 0) ||
-        (s.mhi[2] && i == s.fx - 1))
-      continue;
-    int widx = *p.step0 + p.k;
-    widx = widx < 0 ? 0 : (widx > s.T - 1 ? s.T - 1 : widx);
-    for (int q = 0; q < s.n; ++q) {
-      const int cz = -s.starts[q * 3 + 0];  // the 2D fields' single plane z = 0
-      const int cy = j - s.starts[q * 3 + 1], cx = i - s.starts[q * 3 + 2];
-      if (cz < 0 || cz >= s.sz || cy < 0 || cy >= s.sy || cx < 0 || cx >= s.sx) continue;
-      const int64_t c = ((static_cast<int64_t>(q) * s.sz + cz) * s.sy + cy) * s.sx + cx;
-      v = v + s.coeff[c] * s.wave[static_cast<int64_t>(q) * s.T + widx];
-    }
-  }
-  return v;
-}
 template <typename T, bool kCpml>
 __global__ void __launch_bounds__(kBX * kBY)
 h_phase_tm(PhaseParams p) {
@@ -376,7 +408,7 @@ h_phase_tm(PhaseParams p) {
     float h = coef(p.dec[0], p.dec_st[0], p.dec_s[0], o) * ld<T>(p.tin[0], o) -
               coef(p.scf[0], p.scf_st[0], p.scf_s[0], o) * p.ratio * d;
     if (((m & kLeft) && i == 0) || ((m & kRight) && i == nx)) h = 0.0f;
-    if (p.npsrc > 0) h = tm_sources(p, 0, j, i, h);
+    if (p.psrc[0].n > 0) h = group_add(p, p.psrc[0], 0, j, i, h);
     store_f(static_cast<T*>(p.tout[0]), o, h);
   }
   // Hy (ny+1, nx): corrected(-dEz/dx)
@@ -390,7 +422,7 @@ h_phase_tm(PhaseParams p) {
     float h = coef(p.dec[1], p.dec_st[1], p.dec_s[1], o) * ld<T>(p.tin[1], o) +
               coef(p.scf[1], p.scf_st[1], p.scf_s[1], o) * p.ratio * d;
     if (((m & kBottom) && j == 0) || ((m & kTop) && j == ny)) h = 0.0f;
-    if (p.npsrc > 0) h = tm_sources(p, 1, j, i, h);
+    if (p.psrc[1].n > 0) h = group_add(p, p.psrc[1], 0, j, i, h);
     store_f(static_cast<T*>(p.tout[1]), o, h);
   }
 }
@@ -430,7 +462,7 @@ e_phase_tm(PhaseParams p) {
   if (((m & kBottom) && j == 0) || ((m & kTop) && j == ny) ||
       ((m & kLeft) && i == 0) || ((m & kRight) && i == nx))
     e = 0.0f;
-  if (p.npsrc > 0) e = tm_sources(p, 2, j, i, e);
+  if (p.psrc[2].n > 0) e = group_add(p, p.psrc[2], 0, j, i, e);
   store_f(static_cast<T*>(p.tout[2]), o, e);
 }
 
@@ -484,7 +516,9 @@ void dispatch_tm(hipStream_t s, const PhaseParams& p, int phase) {
 
 void launch_phase3d(hipStream_t s, const PhaseParams& p, int phase, int dtype) {
   BZH_REQUIRE(!p.scf_f16, "f16 coefficient arrays are read only by the fused step");
-  BZH_REQUIRE(p.npsrc == 0, "folded source slabs are for the 2D kernels");
+  BZH_REQUIRE(p.npsrc == 0 || p.step0 != nullptr,
+              "folded source slabs are malformed");
+  BZH_REQUIRE(p.npsrc == 0 || dtype == BZH_F32, "folded source slabs need float32 fields");
   switch (dtype) {
     case BZH_F32: dispatch3d<float>(s, p, phase); break;
     case BZH_BF16: dispatch3d<bf16_t>(s, p, phase); break;
@@ -496,7 +530,7 @@ void launch_phase3d(hipStream_t s, const PhaseParams& p, int phase, int dtype) {
 
 void launch_phase_tm(hipStream_t s, const PhaseParams& p, int phase, int dtype) {
   BZH_REQUIRE(!p.scf_f16, "f16 coefficient arrays are read only by the fused step");
-  BZH_REQUIRE(p.npsrc >= 0 && p.npsrc <= kMaxPhaseSrc && (p.npsrc == 0 || p.step0 != nullptr),
+  BZH_REQUIRE(p.npsrc == 0 || p.step0 != nullptr,
               "folded source slabs are malformed");
   BZH_REQUIRE(p.npsrc == 0 || dtype == BZH_F32, "folded source slabs need float32 fields");
   switch (dtype) {

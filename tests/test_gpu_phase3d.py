@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from oracle import fdtd64 as o
+from tests.test_gpu_pair import _h_sources, _sources
 from tests.test_gpu_parity import _compare_state, _require_gpu, _setup
 
 pytestmark = pytest.mark.gpu
@@ -37,6 +38,24 @@ def test_phase_kernels_parity(grid, cpml, faces, metal, lossy):
     steps = 12
     sim, prog, state, prob, ost = _setup(grid, seed=57, steps=steps, cpml_cells=cpml, faces=faces,
                                          metallic=metal, fused=False, sigma=sigma)
+    state = sim.advance(state, steps)
+    torch.cuda.synchronize()
+    o.run(prob, ost, steps)
+    _compare_state(prog, state, prob, ost)
+
+
+@pytest.mark.parametrize("grid,kw", [((13, 17, 130), dict(cpml_cells=3)), ((9, 28, 64), {}),
+                                     ((11, 14, 67), dict(metallic=("bottom", "left", "back")))])
+def test_folded_sources_parity(grid, kw):
+    """E- and H-timed slabs added by the phase kernels, two of them overlapping
+    on one component and some on masked (metal) faces."""
+    _require_gpu()
+    print(f"case phase3d_sources grid={grid} {kw}", flush=True)
+    steps = 9
+    srcs = _sources(grid, steps) + _h_sources(grid, steps)
+    first = srcs[1]
+    srcs.append(o.Source("Ex", "e", (first.start[0] + 1, 0, 0), first.coeff, first.waveform))
+    sim, prog, state, prob, ost = _setup(grid, seed=58, steps=steps, fused=False, sources=srcs, **kw)
     state = sim.advance(state, steps)
     torch.cuda.synchronize()
     o.run(prob, ost, steps)
