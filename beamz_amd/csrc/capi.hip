@@ -395,7 +395,7 @@ void enqueue(hipStream_t s, const Launch& l) {
     case Kind::kAdjoint: {
       Adjoint2dParams p;
       std::memcpy(&p, l.bytes.data(), sizeof(p));
-      launch_adjoint_step(s, p);
+      launch_adjoint_pass(s, p, l.phase);
       break;
     }
     case Kind::kDft: {
@@ -2591,11 +2591,14 @@ int32_t bzh_adjoint2d_reverse(void* stream, const bzh_adjoint2d* adj, int32_t n_
     if (p.src_profile)
       BZH_REQUIRE(n_last < numel(adj->source_time), "source time factors shorter than the run");
     std::vector<Launch> launches;
+    launches.reserve(2 * static_cast<size_t>(count) + 1);
     for (int c = 0; c < count; ++c) {
       p.n = n_last - c;
       p.slot = slot_last - c;
-      launches.push_back(make_launch(Kind::kAdjoint, 0, BZH_F32, p));
+      launches.push_back(make_launch(Kind::kAdjoint, c == 0 ? kAdjE : kAdjEzE, BZH_F32, p));
+      launches.push_back(make_launch(Kind::kAdjoint, kAdjH, BZH_F32, p));
     }
+    launches.push_back(make_launch(Kind::kAdjoint, kAdjEz, BZH_F32, p));
     graph_cache().run(static_cast<hipStream_t>(stream), launches, (flags & BZH_FLAG_GRAPH_CACHE) != 0);
   });
 }

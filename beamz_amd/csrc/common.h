@@ -505,7 +505,10 @@ struct Adjoint2dParams {
   int32_t slot;              // record slot of step n
   double* grad;              // sum over steps of g * curl, [dy][dx]
 };
-void launch_adjoint_step(hipStream_t s, const Adjoint2dParams& p);
+// Passes of the reverse sweep: E of the first reversed step, then per step H and
+// (Ez of this step with E of the next), Ez alone at the end.
+enum : int32_t { kAdjE = 0, kAdjH, kAdjEzE, kAdjEz };
+void launch_adjoint_pass(hipStream_t s, const Adjoint2dParams& p, int pass);
 // The record launch of one step, as a schedule entry.
 struct AdjointRecordParams {
   Adjoint2dParams p;
