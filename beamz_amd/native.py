@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import threading
 
 import torch
@@ -220,31 +221,55 @@ def status():
     return True, ""
 
 
+# One descriptor's fields in native layout (data, rank, element_type, dims[4]).
+# A call describes about a hundred tensors; writing each with one pack takes
+# half the time of the field-by-field assignments (0.5 against 0.9 us), which
+# was most of the host time of a short call.
+_DESCRIPTOR = struct.Struct("@Pii4q")
+assert _DESCRIPTOR.size == ctypes.sizeof(Buffer)
+_NO_DIMS = (0, 0, 0, 0)
+
+
+class Absent:
+    """A tensor argument without elements, described without allocating one."""
+
+    __slots__ = ("fields",)
+
+    def __init__(self, shape=(0,), dtype=torch.float32):
+        self.fields = (0, len(shape), _DTYPE_CODE[dtype], *(tuple(shape) + _NO_DIMS)[:4])
+
+
+_NONE = Absent()
+
+
+def _describe(into, offset, t):
+    if t is None:
+        t = _NONE
+    if type(t) is Absent:
+        _DESCRIPTOR.pack_into(into, offset, *t.fields)
+        return
+    if not t.is_contiguous():
+        raise HipLaunchError("native buffers must be contiguous")
+    shape = t.shape
+    rank = len(shape)
+    if rank > 4:
+        raise HipLaunchError("native buffers have rank <= 4")
+    _DESCRIPTOR.pack_into(into, offset, 0 if 0 in shape else t.data_ptr(), rank,
+                          _DTYPE_CODE[t.dtype], *shape, *_NO_DIMS[rank:])
+
+
 def buffer(t) -> Buffer:
     """Describe a contiguous tensor (or ``None`` for an empty slot)."""
     b = Buffer()
-    if t is None:
-        b.data = None
-        b.rank = 1
-        b.element_type = F32
-        b.dims[0] = 0
-        return b
-    if not t.is_contiguous():
-        raise HipLaunchError("native buffers must be contiguous")
-    if t.dim() > 4:
-        raise HipLaunchError("native buffers have rank <= 4")
-    b.data = t.data_ptr() if t.numel() else None
-    b.rank = t.dim()
-    b.element_type = _DTYPE_CODE[t.dtype]
-    for d, n in enumerate(t.shape):
-        b.dims[d] = int(n)
+    _describe(b, 0, t)
     return b
 
 
 def buffers(tensors):
     arr = (Buffer * len(tensors))()
+    size = _DESCRIPTOR.size
     for i, t in enumerate(tensors):
-        arr[i] = buffer(t)
+        _describe(arr, i * size, t)
     return arr
 
 

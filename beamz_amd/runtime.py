@@ -20,11 +20,11 @@ from . import _abi as abi
 from . import native
 from .program import CompiledProgram, SimulationState, field_bank
 
-_EMPTY_GROUP = None
-
-
-def _empty(device):
-    return torch.zeros(0, dtype=torch.float32, device=device)
+# Slots without elements: described, not allocated (34 of a 2D call's
+# arguments; as zero-size tensors they took 60 of its 175 us).
+_EMPTY = native.Absent()
+_EMPTY_GROUP = (native.Absent((0, 1, 1, 1)), native.Absent((0, 1)),
+                native.Absent((0, 3), torch.int32))
 
 
 def _metrics(prog, phase):
@@ -33,8 +33,7 @@ def _metrics(prog, phase):
     table = prog.h_metrics if phase == abi.PHASE_H else prog.e_metrics
     if table:
         return tuple(table)
-    e = _empty(prog.device)
-    return (e, e, e)
+    return (_EMPTY, _EMPTY, _EMPTY)
 
 
 def _materials(prog, phase):
@@ -44,19 +43,16 @@ def _materials(prog, phase):
             c[f"{p}_source_x"], c[f"{p}_source_y"], c[f"{p}_source_z"])
 
 
-def _psi_slots(psi, device):
-    slots = list(psi)
-    while len(slots) < abi.CPML_TERM_COUNT:
-        slots.append(_empty(device))
-    return tuple(slots)
+def _psi_slots(psi):
+    return (*psi, *(_EMPTY,) * (abi.CPML_TERM_COUNT - len(psi)))
 
 
 def _cpml_payload(prog, state, phase):
     if phase == abi.PHASE_H:
         return (*_materials(prog, phase), prog.h_meta, *prog.h_term_arrays,
-                *_psi_slots(state.psi_h, prog.device))
+                *_psi_slots(state.psi_h))
     return (*_materials(prog, phase), prog.e_meta, *prog.e_term_arrays,
-            *_psi_slots(state.psi_e, prog.device))
+            *_psi_slots(state.psi_e))
 
 
 def _graph_io(prog: CompiledProgram, state: SimulationState):
@@ -71,15 +67,7 @@ def _graph_io(prog: CompiledProgram, state: SimulationState):
 
 
 def _source_group_arguments(prog):
-    out = []
-    for g in prog.source_groups:
-        if g is None:
-            dev = prog.device
-            out += [torch.zeros((0, 1, 1, 1), device=dev), torch.zeros((0, 1), device=dev),
-                    torch.zeros((0, 3), dtype=torch.int32, device=dev)]
-        else:
-            out += list(g)
-    return tuple(out)
+    return tuple(t for g in prog.source_groups for t in (_EMPTY_GROUP if g is None else g))
 
 
 def _program_attrs(prog, nsteps, layout, monitor_count=0):
@@ -291,7 +279,7 @@ def step_kernel_name(prog, pairs=False):
     if uses_two_banks(prog):
         # one pair launch runs the general and the core bodies
         return "pair_step" if pairs else "fused_interior+fused_edge"
-    return "h_phase_3d+e_phase_3d" if prog.is_3d else "h_phase_tm+e_phase_tm"
+    return "phase_3d" if prog.is_3d else "h_phase_tm+e_phase_tm"
 
 
 def time_step_kernel(state, prog, *, launches=20, stream=None):
@@ -305,7 +293,7 @@ def time_step_kernel(state, prog, *, launches=20, stream=None):
         stop = torch.cuda.Event(enable_timing=True)
         if uses_two_banks(prog):
             layout_state = with_workspace(layout_state)
-            args = (*_temporal_io(prog, layout_state), *_source_group_arguments_empty(prog),
+            args = (*_temporal_io(prog, layout_state), *_EMPTY_GROUP * abi.SOURCE_GROUP_COUNT,
                     layout_state.current_step)
             attrs = _program_attrs(prog, 4, abi.PROGRAM_LAYOUT_SOURCE_TEMPORAL_CPML)
             attrs.coincident_source_group_mask = 0
@@ -320,15 +308,6 @@ def time_step_kernel(state, prog, *, launches=20, stream=None):
         stop.record(stream)
     torch.cuda.synchronize()
     return start.elapsed_time(stop) / (4 * launches)
-
-
-def _source_group_arguments_empty(prog):
-    dev = prog.device
-    out = []
-    for _ in range(abi.SOURCE_GROUP_COUNT):
-        out += [torch.zeros((0, 1, 1, 1), device=dev), torch.zeros((0, 1), device=dev),
-                torch.zeros((0, 3), dtype=torch.int32, device=dev)]
-    return tuple(out)
 
 
 # ---- descriptor-level entry points (cuda/src/launch.h:12-77) -----------------
@@ -360,12 +339,12 @@ def _phase_launch(prog, phase, targets, sources, psi, out_targets, out_psi):
     if prog.cpml_enabled:
         meta = prog.h_meta if phase == abi.PHASE_H else prog.e_meta
         arrays = prog.h_term_arrays if phase == abi.PHASE_H else prog.e_term_arrays
-        ins += [meta, *arrays[:18], *_psi_slots(psi, prog.device)]
+        ins += [meta, *arrays[:18], *_psi_slots(psi)]
     _fill(ln.inputs, ins + [None] * (37 - len(ins)))
     _fill(ln.metrics, _metrics(prog, phase))
     outs = [*out_targets]
     if prog.cpml_enabled:
-        outs += list(_psi_slots(out_psi, prog.device))
+        outs += list(_psi_slots(out_psi))
     _fill(ln.outputs, outs + [None] * (9 - len(outs)))
     return ln
 
