@@ -319,23 +319,39 @@ class PreparedProgram:
     object issues the same call again on the current stream.  For loops that
     step one state many times in short chunks, where building the array
     (a few tens of tensors) costs far more host time than the launch.  It
-    holds the tensors; they must keep their storage while it is used."""
+    holds the tensors; they must keep their storage while it is used.
+    ``scratch``: those of them that nothing else holds, allocated on the
+    current stream."""
 
-    def __init__(self, args, attrs: ProgramAttrs):
+    def __init__(self, args, attrs: ProgramAttrs, scratch=()):
         self._args = tuple(args)
         self._arr = buffers(self._args)
         self._attrs = attrs
+        self._scratch = [t for t in scratch if t.is_cuda]
+        self._streams = {current_stream_handle().value or 0} if self._scratch else set()
+
+    def _stream(self, stream):
+        """The call's stream; on another one than the scratch was allocated on,
+        dropping this object must not hand the scratch on before its work."""
+        s = current_stream_handle() if stream is None else stream
+        handle = getattr(s, "value", s) or 0
+        if self._scratch and handle not in self._streams:
+            self._streams.add(handle)
+            on = torch.cuda.ExternalStream(handle) if handle else torch.cuda.default_stream()
+            for t in self._scratch:
+                t.record_stream(on)
+        return s
 
     def __call__(self, stream=None):
         lib = library()
-        s = current_stream_handle() if stream is None else stream
+        s = self._stream(stream)
         _check(lib.bzh_program(s, self._arr, len(self._args), ctypes.byref(self._attrs)), lib)
 
     def recompute(self, adj, nsteps, slot, stream=None):
         """The call for ``nsteps`` steps that also records each step's forward
         curl of ``adj`` from record slot ``slot`` (``bzh_adjoint2d_recompute``)."""
         lib = library()
-        s = current_stream_handle() if stream is None else stream
+        s = self._stream(stream)
         attrs = ProgramAttrs.from_buffer_copy(self._attrs)
         attrs.nsteps = int(nsteps)
         _check(lib.bzh_adjoint2d_recompute(s, self._arr, len(self._args), ctypes.byref(attrs),

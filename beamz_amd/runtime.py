@@ -13,6 +13,7 @@ the same state object is returned.
 from __future__ import annotations
 
 import ctypes
+import weakref
 
 import torch
 
@@ -149,13 +150,40 @@ def _temporal_io(prog, state):
     return (*_graph_io(prog, state), *state.fields_b)
 
 
+class Workspace2D(tuple):
+    """A 2D state's launch scratch in its second-bank slot: one tensor, used by
+    the state that holds ``ez`` and on the stream it was allocated on.  A state
+    forked with tensors of its own, or a call on another stream, gets another
+    one, so that two forks on two streams never write the same scratch, and a
+    dropped one is reused only behind the work that was queued on it.  Its
+    contents do not outlive a call: copies and pickles leave it out."""
+
+    def __new__(cls, tensor, ez, stream):
+        self = super().__new__(cls, (tensor,))
+        self.ez = weakref.ref(ez)
+        self.stream = stream
+        return self
+
+    def fits(self, ez, stream, floats):
+        return self.ez() is ez and self.stream == stream and self[0].numel() >= floats
+
+    def __reduce__(self):
+        return torch.Size, ((),)  # an empty tuple that ``weights_only`` loading accepts
+
+
 def with_workspace_2d(state, prog):
     """The state with the 2D program's multi-step workspace in its second-bank
-    slot (allocated on first use; its contents do not outlive a call)."""
+    slot (:class:`Workspace2D`), allocated where the state has none of its own
+    for the current stream."""
     n = prog.workspace_floats
-    if n == 0 or prog.is_3d or (len(state.fields_b) == 1 and state.fields_b[0].numel() >= n):
+    if n == 0 or prog.is_3d:
         return state
-    return state._replace(fields_b=(torch.empty(n, dtype=torch.float32, device=prog.device),))
+    stream = torch.cuda.current_stream().cuda_stream if prog.device.type == "cuda" else 0
+    held = state.fields_b
+    if isinstance(held, Workspace2D) and held.fits(state.ez, stream, n):
+        return state
+    tensor = torch.empty(n, dtype=torch.float32, device=prog.device)
+    return state._replace(fields_b=Workspace2D(tensor, state.ez, stream))
 
 
 def _workspace_args(state, prog):
@@ -245,13 +273,14 @@ def prepare_chunk(state, prog, nsteps):
         return native.PreparedProgram(
             (*_graph_io(prog, state), *_monitor_tail(state, prog, False), *ws),
             _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_MONITOR_IN_PLACE,
-                           monitor_count=len(prog.monitors)))
+                           monitor_count=len(prog.monitors)), scratch=ws)
     if any(g is not None for g in prog.source_groups):
         return native.PreparedProgram(
             (*_graph_io(prog, state), *_source_group_arguments(prog), state.current_step, *ws),
-            _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_SOURCE_IN_PLACE))
+            _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_SOURCE_IN_PLACE), scratch=ws)
     layout = abi.PROGRAM_LAYOUT_CPML_IN_PLACE if prog.cpml_enabled else abi.PROGRAM_LAYOUT_YEE_IN_PLACE
-    return native.PreparedProgram((*_graph_io(prog, state), *ws), _program_attrs(prog, nsteps, layout))
+    return native.PreparedProgram((*_graph_io(prog, state), *ws),
+                                  _program_attrs(prog, nsteps, layout), scratch=ws)
 
 
 GRAPH_MAX_STEPS = 256  # execute.py:64

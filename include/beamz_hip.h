@@ -231,7 +231,8 @@ int32_t bzh_streamed(void* stream, const bzh_buffer* args, int32_t nargs,
  * device workspace (rank 1): with room for a second bank of Ez, Hx, Hy and the
  * four CPML memories, each rounded up to 64 floats, and for 32 steps of the
  * boxes' cells, float32 programs run several steps per launch; the results
- * are bitwise the same and the workspace's contents are undefined after. */
+ * are bitwise the same and the workspace's contents are undefined after.  Calls
+ * that may overlap in time need workspaces of their own. */
 int32_t bzh_program(void* stream, const bzh_buffer* args, int32_t nargs,
                     const bzh_program_attrs* attrs);
 
