@@ -637,6 +637,25 @@ void add_source_launches(std::vector<Launch>& out, const SourceGroupIn& grp, int
   }
 }
 
+// Does a 3D phase add this group's slabs itself (fold_phase_sources)?  Folded,
+// every wave of the grid tests every slab, and the waves on the slab's rows of
+// cells, whatever their x, also read its waveform; launched, a slab costs a
+// launch, its rows (strided) and its cells.  The two costs in us per step and
+// slab, millions of nodes, rows and cells, fitted to (folded / launched, with
+// the hit fraction of the rows): one cell and sheets across x at 65x113x161
+// nodes 0.8 / 1.8 and 2.2 / 2.8 (0.48), at 73x121x201 1.3 / 1.8 and 4.1 / 3.0
+// (0.52), at 97x161x241 2.4 / 2.1 and 9.9 / 3.9 (0.63), at 193x257x257 9.5 / 2.2
+// and 30 / 9.7 (0.79); slabs of 0.7 M cells at 73x121x201 3.7 / 4.7, of 8.5 M at
+// 193x257x257 40 / 32.
+bool fold_group(const Grid& g, const SourceGroupIn& grp) {
+  const bzh_buffer& c = *grp.coeffs;
+  if (!g.is3d || c.rank != 4) return true;
+  const double grid_rows = 1e-6 * (g.nz + 1) * (g.ny + 1), nodes = grid_rows * (g.nx + 1);
+  const double rows = 1e-6 * c.dims[1] * c.dims[2], cells = rows * c.dims[3];
+  const double folded = nodes * (0.75 + 2.1 * std::min(rows / grid_rows, 1.0)) + 1.2 * cells;
+  return folded <= 2.1 + 190.0 * rows + 2.6 * cells;
+}
+
 // Fold a timed source group into a phase launch (PhaseParams::psrc): the
 // checks of add_source_launches, then the group's slabs, summed per cell in
 // declaration order inside the kernel.
@@ -1894,11 +1913,10 @@ bool run_program(hipStream_t s, ProgramIn& in) {
   }
 
   const Kind pk = g.is3d ? Kind::kPhase3d : Kind::kPhaseTm;
-  // float32 programs fold their timed source slabs into the phase launches: a
-  // launch of its own costs 5 us, as much as a small phase (2D: three launches
-  // per step instead of five, H, E and the DFT sample; 64x112x160 with
-  // electric and magnetic sheets: 51 -> 48.5 us per step); the groups that do
-  // not fit keep their source launches
+  // float32 programs fold their timed source slabs into the phase launches (2D:
+  // three launches per step instead of five, H, E and the DFT sample; 3D: the
+  // groups where it pays, fold_group; 64x112x160 with electric and magnetic
+  // sheets: 51 -> 48.5 us per step); the others keep their source launches
   bool fold = g.dtype == BZH_F32 && step0 != nullptr;
   for (int c = 0; c < 3 && fold && !g.is3d; ++c) {
     if (3 + c < in.ngroups && group_slabs(in.groups[3 + c]) > 0 && c == 2) fold = false;  // (no Hz in TMxy)
@@ -2001,18 +2019,20 @@ bool run_program(hipStream_t s, ProgramIn& in) {
       if (fold) {
         // the H-timed slabs and the E-timed ones run inside the phase launches
         for (int c = 0; c < 3 && 3 + c < in.ngroups; ++c)
-          fold_phase_sources(hp, in.groups[3 + c], c, kHx + c, nxt, g, in.metallic, step0, k);
+          if (fold_group(g, in.groups[3 + c]))
+            fold_phase_sources(hp, in.groups[3 + c], c, kHx + c, nxt, g, in.metallic, step0, k);
         for (int c = 0; c < 3 && 6 + c < in.ngroups; ++c)
-          fold_phase_sources(ep, in.groups[6 + c], c, kEx + c, nxt, g, in.metallic, step0, k);
+          if (fold_group(g, in.groups[6 + c]))
+            fold_phase_sources(ep, in.groups[6 + c], c, kEx + c, nxt, g, in.metallic, step0, k);
       }
       launches.push_back(make_launch(pk, BZH_PHASE_H, g.dtype, hp));
-      if (!fold)
-        for (int c = 0; c < 3 && 3 + c < in.ngroups; ++c)
+      for (int c = 0; c < 3 && 3 + c < in.ngroups; ++c)
+        if (!fold || !fold_group(g, in.groups[3 + c]))
           add_source_launches(launches, in.groups[3 + c], 1, c, nxt, g, in.metallic, step0, k);
       launches.push_back(make_launch(pk, BZH_PHASE_E, g.dtype, ep));
     }
-    if (fused || !fold)
-      for (int c = 0; c < 3 && 6 + c < in.ngroups; ++c)
+    for (int c = 0; c < 3 && 6 + c < in.ngroups; ++c)
+      if (fused || !fold || !fold_group(g, in.groups[6 + c]))
         add_source_launches(launches, in.groups[6 + c], 2, c, nxt, g, in.metallic, step0, k);
     if (in.has_monitors) add_dft(k, nxt);
     if (in.record != nullptr) {

@@ -60,3 +60,21 @@ def test_folded_sources_parity(grid, kw):
     torch.cuda.synchronize()
     o.run(prob, ost, steps)
     _compare_state(prog, state, prob, ost)
+
+
+def test_launched_and_folded_sources_parity():
+    """A grid where a source over most rows gets a launch of its own and small
+    sources run inside the phase kernels, both on one phase."""
+    _require_gpu()
+    grid, steps = (96, 128, 136), 6
+    print(f"case phase3d_sources grid={grid}", flush=True)
+    srcs = _sources(grid, steps) + _h_sources(grid, steps)
+    wave = srcs[0].waveform
+    srcs += [o.Source("Ey", "e", (2, 3, 9), np.full((90, 120, 1), 0.05), wave),
+             o.Source("Hx", "h", (1, 2, 30), np.full((92, 122, 2), 1e-4), wave),
+             o.Source("Ex", "e", (50, 60, 70), np.full((2, 1, 3), 0.1), wave)]
+    sim, prog, state, prob, ost = _setup(grid, seed=59, steps=steps, fused=False, sources=srcs, cpml_cells=4)
+    state = sim.advance(state, steps)
+    torch.cuda.synchronize()
+    o.run(prob, ost, steps)
+    _compare_state(prog, state, prob, ost)
