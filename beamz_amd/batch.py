@@ -30,6 +30,11 @@ from .program import CompiledProgram
 # 16: two rows per lane (16-wave tiles: fewer tiles than CUs), 32: four (8 and
 # 64 are taken as these)
 TILE_ROWS = (16, 32)
+# steps of a tuning call: a multiple of these deals out whole launches of 8 steps
+# and of 6 (large batches), as the calls of ``advance`` run them.  The tile
+# height that is faster depends on that depth (a call of 6 steps runs launches
+# of 3, whose tiles own 58 x 26 cells instead of 48 x 16).
+TUNING_STEPS = 48
 MAX_SOURCES = 4
 _TUNED: dict = {}
 
@@ -214,11 +219,11 @@ class BatchedSimulation2D:
 
 
 def autotune(batch: BatchedSimulation2D, *, steps=6, candidates=None, verbose=False):
-    """Pick ``tile_rows`` of ``batch`` by timing each candidate for a few steps
-    on a scratch state; the choice is cached per batch signature (grid shapes
-    and CPML thickness).  Returns ``(tile_rows, workgroups, timings)``; every
+    """Pick ``tile_rows`` of ``batch`` by timing each candidate for at least
+    ``steps`` steps (whole launches, ``TUNING_STEPS``) on a scratch state; the
+    choice is cached per batch signature (grid shapes and CPML thickness).  Returns ``(tile_rows, workgroups, timings)``; every
     tile is its own workgroup, so ``workgroups`` changes nothing."""
-    steps = max(2, steps + steps % 2)  # even: the banks end where they start
+    steps = -(-max(int(steps), 1) // TUNING_STEPS) * TUNING_STEPS
     key = batch.signature()
     if key in _TUNED:
         batch.tile_rows, batch.workgroups = _TUNED[key][:2]
