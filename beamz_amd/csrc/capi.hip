@@ -2202,25 +2202,23 @@ void copy_psi_workspace(hipStream_t s, const bzh_buffer* args, int nargs) {
 }
 
 // ---- batched 2D simulations ---------------------------------------------------
-// Device copies of the descriptor table and of the item list, keyed on their
-// bytes.  They are kept for the life of the process: a captured graph refers
-// to them.
-template <typename V>
-const void* upload_cached(const std::vector<V>& host) {
+// Device copies of the members' descriptors, keyed on their bytes.  They are
+// kept for the life of the process: a captured graph refers to them.
+const TmSim* upload_sims(const std::vector<TmSim>& sims) {
   static std::mutex mu;
   static std::map<std::string, void*> cache;
   int device = 0;
   BZH_HIP(hipGetDevice(&device));
   std::string key(reinterpret_cast<const char*>(&device), sizeof(device));
-  key.append(reinterpret_cast<const char*>(host.data()), host.size() * sizeof(V));
+  key.append(reinterpret_cast<const char*>(sims.data()), sims.size() * sizeof(TmSim));
   std::lock_guard<std::mutex> lock(mu);
-  auto it = cache.find(key);
-  if (it != cache.end()) return it->second;
+  const auto it = cache.find(key);
+  if (it != cache.end()) return static_cast<const TmSim*>(it->second);
   void* d = nullptr;
-  BZH_HIP(hipMalloc(&d, std::max<size_t>(host.size() * sizeof(V), 16)));
-  BZH_HIP(hipMemcpy(d, host.data(), host.size() * sizeof(V), hipMemcpyHostToDevice));
+  BZH_HIP(hipMalloc(&d, sims.size() * sizeof(TmSim)));
+  BZH_HIP(hipMemcpy(d, sims.data(), sims.size() * sizeof(TmSim), hipMemcpyHostToDevice));
   cache[key] = d;
-  return d;
+  return static_cast<const TmSim*>(d);
 }
 
 float* f32_ptr(const bzh_buffer& b, int64_t expect, const std::string& what) {
@@ -2298,23 +2296,51 @@ TmSim describe_sim2d(const bzh_sim2d& in, int index) {
   return d;
 }
 
-// The tiles of every member at T steps per launch, largest simulations first,
-// row-major within one.
-std::vector<int4> batch_tiles(const std::vector<TmSim>& sims, int T) {
+// The tiles of every member, largest simulations first, row-major within one,
+// on the device: a list for each of 1 .. T steps per launch, so that the calls
+// of any step count after the first of a set of shapes allocate and copy
+// nothing (a caller may capture them).  Kept, like the descriptors.
+struct BatchTiles {
+  const int4* at[kTmMaxSteps + 1];
+  int32_t n[kTmMaxSteps + 1];
+};
+const BatchTiles& upload_tiles(const std::vector<TmSim>& sims, int T) {
+  static std::mutex mu;
+  static std::map<std::vector<int>, BatchTiles> cache;   // (its nodes stay in place)
+  int device = 0;
+  BZH_HIP(hipGetDevice(&device));
+  std::vector<int> key{device, T};
+  for (const TmSim& d : sims) {
+    key.push_back(d.ny);
+    key.push_back(d.nx);
+  }
+  std::lock_guard<std::mutex> lock(mu);
+  const auto it = cache.find(key);
+  if (it != cache.end()) return it->second;
   std::vector<int> order(sims.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = static_cast<int>(i);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
     return static_cast<int64_t>(sims[x].ny) * sims[x].nx > static_cast<int64_t>(sims[y].ny) * sims[y].nx;
   });
-  const int cols = 64 - 2 * T, rows = kTmRows - 2 * T;
+  BatchTiles out = {};
   std::vector<int4> tiles;
-  for (int i : order) {
-    const int ty = (sims[i].ny + rows) / rows, tx = (sims[i].nx + cols) / cols;
-    for (int r = 0; r < ty; ++r)
-      for (int c = 0; c < tx; ++c) tiles.push_back(make_int4(i, r, c, 0));
+  size_t first[kTmMaxSteps + 1] = {};
+  for (int t = 1; t <= T; ++t) {
+    first[t] = tiles.size();
+    const int cols = 64 - 2 * t, rows = kTmRows - 2 * t;
+    for (int i : order) {
+      const int ty = (sims[i].ny + rows) / rows, tx = (sims[i].nx + cols) / cols;
+      for (int r = 0; r < ty; ++r)
+        for (int c = 0; c < tx; ++c) tiles.push_back(make_int4(i, r, c, 0));
+    }
+    BZH_REQUIRE(tiles.size() - first[t] < (size_t{1} << 31), "too many tiles");
+    out.n[t] = static_cast<int32_t>(tiles.size() - first[t]);
   }
-  BZH_REQUIRE(tiles.size() < (size_t{1} << 31), "too many tiles");
-  return tiles;
+  void* d = nullptr;
+  BZH_HIP(hipMalloc(&d, tiles.size() * sizeof(int4)));
+  BZH_HIP(hipMemcpy(d, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
+  for (int t = 1; t <= T; ++t) out.at[t] = static_cast<const int4*>(d) + first[t];
+  return cache.emplace(std::move(key), out).first->second;
 }
 
 void run_batch2d(hipStream_t s, const bzh_sim2d* sims, int nsims, const bzh_buffer* step,
@@ -2338,19 +2364,17 @@ void run_batch2d(hipStream_t s, const bzh_sim2d* sims, int nsims, const bzh_buff
   if ((a.nsteps - n) % 2 != 0) ++n;
   TmBatchParams p;
   std::memset(&p, 0, sizeof(p));
-  p.sims = static_cast<const TmSim*>(upload_cached(desc));
+  p.sims = upload_sims(desc);
+  const BatchTiles& lists = upload_tiles(desc, T);
   p.step0 = static_cast<const int32_t*>(step->data);
   p.rpt = a.tile_rows <= 16 ? 2 : 4;
   std::vector<Launch> launches;
   int done = 0;
   for (int i = 0; i < n; ++i) {
     const int steps = a.nsteps / n + (i < a.nsteps % n ? 1 : 0);
-    if (steps != p.T) {
-      const std::vector<int4> list = batch_tiles(desc, steps);
-      p.tiles = static_cast<const int4*>(upload_cached(list));
-      p.ntiles = static_cast<int>(list.size());
-      p.T = steps;
-    }
+    p.T = steps;
+    p.tiles = lists.at[steps];
+    p.ntiles = lists.n[steps];
     p.k = done;
     p.bank = i & 1;
     launches.push_back(make_launch(Kind::kBatch2d, 0, BZH_F32, p));
