@@ -10,8 +10,10 @@ is captured once as a hipGraph and replayed.
 
 Each member is lowered exactly like a single simulation (``program.py``):
 same coefficients, CPML profiles, PEC faces and pre-E soft sources, so a
-member of a batch reproduces the same simulation run alone.  The rows a lane
-holds (``tile_rows``) are chosen by :func:`autotune` on the actual batch.
+member of a batch with CPML has the fields of the same simulation run alone, bit
+for bit; without CPML a lone run rounds each curl once (a fused operation), a
+member its two terms first.  The rows a lane holds (``tile_rows``) are chosen by
+:func:`autotune` on the actual batch.
 """
 
 from __future__ import annotations
