@@ -10,6 +10,7 @@
 // The DFT accumulators and their phase factors are float64: the phase
 // 2*pi*f*t_phys is evaluated in float64 from t_phys = t + (k + 1) dt.
 
+#include <algorithm>
 #include <climits>
 
 #include "common.h"
@@ -405,7 +406,7 @@ void dft_dispatch(hipStream_t s, const DftParams& p) {
     grid.y = p.pair != 0 ? 2 : 1;
     hipLaunchKernelGGL((dft_stage_kernel<T>), grid, block, 0, s, p);
   } else if (p.mode == 2) {
-    grid.y = (p.Fmax + kFt - 1) / kFt;
+    grid.y = std::max(1, (p.Fmax + kFt - 1) / kFt);  // (no frequency: nothing to add)
     if (p.acc_f64) hipLaunchKernelGGL((dft_flush_kernel<double>), grid, block, 0, s, p);
     else hipLaunchKernelGGL((dft_flush_kernel<float>), grid, block, 0, s, p);
   } else {
@@ -515,7 +516,7 @@ void launch_dft_capture(hipStream_t s, const DftCapParams& p) {
   BZH_REQUIRE(d.M <= kMaxMonBoxes && d.nk >= 1 && d.nk <= kDftMaxSlots && p.cap != nullptr,
               "captured DFT is malformed");
   const dim3 block(kDftBlock),
-      grid((d.Pmax + kDftBlock - 1) / kDftBlock, (d.Fmax + kFt - 1) / kFt, d.M * 6);
+      grid((d.Pmax + kDftBlock - 1) / kDftBlock, std::max(1, (d.Fmax + kFt - 1) / kFt), d.M * 6);
   if (d.acc_f64) hipLaunchKernelGGL((dft_capture_kernel<double>), grid, block, 0, s, p);
   else hipLaunchKernelGGL((dft_capture_kernel<float>), grid, block, 0, s, p);
   BZH_HIP(hipGetLastError());
