@@ -381,8 +381,8 @@ def compile_program(permittivity, resolution, dt, *, boundaries=(), sources=(), 
         h_term_arrays=h_arrays, e_term_arrays=e_arrays, source_groups=groups,
         coincident_mask=coincident, monitors=compiled, packed_monitors=packed,
         monitor_boxes=boxes,
-        workspace_floats=0 if is_3d else workspace_floats_2d(shapes, cpml, field_dtype, psi_dtype,
-                                                             metric_kind, boxes),
+        workspace_floats=0 if is_3d or (cpml is not None and thickness == 0) else workspace_floats_2d(
+            shapes, cpml, field_dtype, psi_dtype, metric_kind, boxes, groups),
         device=device, field_dtype=field_dtype, psi_dtype=psi_dtype, flags=int(flags), eps_cells=eps,
         eps_site=eps_site, metric_kind=metric_kind, h_metrics=h_metrics, e_metrics=e_metrics,
         cell_grid=cell_grid if metric_kind else None)
@@ -393,14 +393,21 @@ def compile_program(permittivity, resolution, dt, *, boundaries=(), sources=(), 
 # read more run the per-phase schedule
 CAPTURE_SLOTS = 32
 MAX_CAPTURE_CELLS = 1 << 20
+# monitors and source slabs of a multi-step launch (kMaxMonBoxes, kMaxTmSlabs)
+MAX_CAPTURE_MONITORS = 8
+MAX_STEP_SLABS = 12
 
 
-def workspace_floats_2d(shapes, cpml, field_dtype, psi_dtype, metric_kind, boxes):
+def workspace_floats_2d(shapes, cpml, field_dtype, psi_dtype, metric_kind, boxes, groups=()):
     """Floats of a 2D program's multi-step workspace (``bzh_program``): a
     second bank of the fields and CPML memories, each rounded up to 64 floats,
     and 32 steps of the monitored cells; 0 where the library takes the
     per-phase schedule anyway."""
     if field_dtype != torch.float32 or psi_dtype != torch.float32 or metric_kind:
+        return 0
+    if sum(g[0].shape[0] for g in groups if g is not None) > MAX_STEP_SLABS:
+        return 0
+    if boxes is not None and boxes.shape[0] > MAX_CAPTURE_MONITORS:
         return 0
     sizes = [int(np.prod(s)) for s in shapes.values()]
     for t in (cpml.h_terms + cpml.e_terms) if cpml is not None else ():

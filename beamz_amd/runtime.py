@@ -308,35 +308,42 @@ def step_kernel_name(prog, pairs=False):
     if uses_two_banks(prog):
         # one pair launch runs the general and the core bodies
         return "pair_step" if pairs else "fused_interior+fused_edge"
-    return "phase_3d" if prog.is_3d else "h_phase_tm+e_phase_tm"
+    if prog.is_3d:
+        return "phase_3d"
+    return "tm_steps" if prog.workspace_floats else "h_phase_tm+e_phase_tm"
 
 
 def time_step_kernel(state, prog, *, launches=20, stream=None):
     """Average device time of one bare field step (no sources or monitors),
     measured with events on ``stream``: four steps per call (two pair launches
-    where the pair kernel runs) so the banks return to their starting roles."""
+    where the pair kernel runs) so the banks return to their starting roles, 48
+    (launches of eight or six steps) where a 2D program runs several per launch."""
     stream = stream or torch.cuda.current_stream()
     with torch.cuda.stream(stream):
         layout_state = state
+        steps = 4
         start = torch.cuda.Event(enable_timing=True)
         stop = torch.cuda.Event(enable_timing=True)
         if uses_two_banks(prog):
             layout_state = with_workspace(layout_state)
             args = (*_temporal_io(prog, layout_state), *_EMPTY_GROUP * abi.SOURCE_GROUP_COUNT,
                     layout_state.current_step)
-            attrs = _program_attrs(prog, 4, abi.PROGRAM_LAYOUT_SOURCE_TEMPORAL_CPML)
+            attrs = _program_attrs(prog, steps, abi.PROGRAM_LAYOUT_SOURCE_TEMPORAL_CPML)
             attrs.coincident_source_group_mask = 0
         else:
             layout = abi.PROGRAM_LAYOUT_CPML_IN_PLACE if prog.cpml_enabled else abi.PROGRAM_LAYOUT_YEE_IN_PLACE
-            args = _graph_io(prog, layout_state)
-            attrs = _program_attrs(prog, 4, layout)
+            layout_state = with_workspace_2d(layout_state, prog)
+            ws = _workspace_args(layout_state, prog)
+            steps = 48 if ws else steps
+            args = (*_graph_io(prog, layout_state), *ws)
+            attrs = _program_attrs(prog, steps, layout)
         native.call_program(args, attrs)  # warm (captures the graph)
         start.record(stream)
         for _ in range(launches):
             native.call_program(args, attrs)
         stop.record(stream)
     torch.cuda.synchronize()
-    return start.elapsed_time(stop) / (4 * launches)
+    return start.elapsed_time(stop) / (steps * launches)
 
 
 # ---- descriptor-level entry points (cuda/src/launch.h:12-77) -----------------
