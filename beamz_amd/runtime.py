@@ -156,7 +156,8 @@ class Workspace2D(tuple):
     forked with tensors of its own, or a call on another stream, gets another
     one, so that two forks on two streams never write the same scratch, and a
     dropped one is reused only behind the work that was queued on it.  Its
-    contents do not outlive a call: copies and pickles leave it out."""
+    contents do not outlive a call: copies and pickles leave it out.  A caller's
+    graph refers to the scratch of the state that the captured call returned."""
 
     def __new__(cls, tensor, ez, stream):
         self = super().__new__(cls, (tensor,))

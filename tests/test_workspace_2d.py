@@ -86,3 +86,46 @@ def test_forks_on_two_streams_match_lone_runs():
         for a, b in zip((got.hx, got.hy, got.ez, *got.psi_h, *got.psi_e),
                         (ref.hx, ref.hy, ref.ez, *ref.psi_h, *ref.psi_e)):
             assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("warm", [False, True])
+def test_captured_calls_replay(warm):
+    """A call in a caller's graph, with and without a warm-up on its stream."""
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a GPU")
+    native.library()
+    print(f"case captured 2D call warm={warm}", flush=True)
+    sim = _simulation(150, 230)
+    prog = sim.compile()
+    rng = np.random.default_rng(6)
+    fields = {c.lower(): rng.normal(size=prog.shapes[c]) * (1.0 if c[0] == "E" else 1 / 377)
+              for c in prog.shapes}
+
+    def chunk(state):
+        state = runtime.run_chunk(state, prog, 9)
+        state.current_step.add_(9)
+        state.t.add_(9 * prog.dt)
+        return state
+
+    got, want = sim.initial_state(fields), sim.initial_state(fields)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    if warm:
+        with torch.cuda.stream(stream):
+            got = chunk(got)
+        want = chunk(want)
+        torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        held = chunk(got)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        want = chunk(want)
+        torch.cuda.synchronize()
+        for a, b in zip((held.hx, held.hy, held.ez, *held.psi_h, *held.psi_e),
+                        (want.hx, want.hy, want.ez, *want.psi_h, *want.psi_e)):
+            assert torch.equal(a, b)
+        for a, b in ((held.dft_re, want.dft_re), (held.dft_im, want.dft_im), (held.dft_w, want.dft_w)):
+            assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
