@@ -169,7 +169,7 @@ def run_batched(args):
     torch.cuda.synchronize()
     stream = torch.cuda.Stream()
     with torch.cuda.stream(stream):
-        if args.tile_rows and args.workgroups:
+        if args.tile_rows:
             batch.tile_rows, batch.workgroups = tr, wg = args.tile_rows, args.workgroups
             timings = {}
         else:
@@ -456,8 +456,8 @@ def main():
     ap.add_argument("--per-phase", action="store_true", help="use the per-phase kernels")
     ap.add_argument("--chunk", type=int, default=256)
     ap.add_argument("--tile-rows", type=int, default=0,
-                    help="batched2d: 16 or 32 (with --workgroups, skips the autotuner)")
-    ap.add_argument("--workgroups", type=int, default=0, help="batched2d: unused by the kernel; any non-zero value")
+                    help="batched2d: 16 or 32 (skips the autotuner)")
+    ap.add_argument("--workgroups", type=int, default=0, help="batched2d: reported only (every tile is its own workgroup)")
     ap.add_argument("--workload", default="3d", choices=("3d", "waveguide3d", "batched2d", "adjoint2d"),
                     help="3d: the 1024x512x256 Yee+CPML step (default); waveguide3d: the 512x256x128 "
                          "silicon strip; batched2d: the 64-simulation "
