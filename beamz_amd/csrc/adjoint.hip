@@ -21,12 +21,13 @@
 //   adj_h:  aHy += ghost-x-diff^T(A0), aHx += ghost-y-diff^T(A1); then the H
 //           transposes: aH <- dH g_h, B = a_d/dx with the H-term recurrences
 //   adj_ez: aEz += forward-diff^T(Bx, By)
-// adj_ez of one step and adj_e of the next both touch a cell's own aEz only, so
-// they share a launch: two launches per step.  At 300 x 300 a pass moves 2 MB and
-// takes 3.6 to 3.9 us, most of it the launch; a 400-step gradient took 10.0 ms
-// with three launches per step and 9.1 ms with two.
 // where W is the monitor's adjoint source profile and c_n its time factor for
 // step n, and curl_n the forward (d0' - d1') recorded over the design region.
+//
+// adj_ez of one step and adj_e of the next both touch a cell's own aEz only, so
+// they share a launch: two launches per step.  At 300 x 300 a pass moves 2 MB and
+// takes 4.1 to 4.7 us, most of it the launch; a 400-step gradient took 10.0 ms
+// with three launches per step and 9.1 ms with two.
 
 #include "common.h"
 

@@ -1424,8 +1424,12 @@ bool metrics_empty(const PhaseIn& ph) {
 // flux lines and a line source: 200x400 (117 tiles of 48 x 16) 15.0 / 8 with
 // two rows and 18.4 / 8 with four, 1201x1603 (2584 tiles) 77.7 / 8 and
 // 55.4 / 8, there 39.2 / 6 and 28.8 / 4 with four rows; 450x450 (290 tiles)
-// measured equal, 600x600 (494) 8 % faster with four rows.  BZH_TM_T overrides
-// the steps.
+// measured equal, 600x600 (494) 8 % faster with four rows.  Where eight steps
+// give way to six, us per step in calls of 96 steps, 8 / 6: 1128 tiles 5.46 /
+// 5.88, 1568 6.71 / 6.58, 1891 7.28 / 7.07, 2312 8.00 / 7.67, 6930 17.1 / 15.5;
+// batches 767 3.14 / 3.51, 1400 4.47 / 4.34, 2363 6.70 / 5.96, 5873 12.8 / 11.3.
+// (From 1400 tiles to the line the two are within 4 %.)  BZH_TM_T overrides the
+// steps.
 struct TmShape {
   int T, rpt;
 };

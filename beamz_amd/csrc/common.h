@@ -97,15 +97,11 @@ struct DevTerm {
   int32_t psi_bf16;   // psi stored as bf16
 };
 
-// Fields of one phase: three targets (updated in place, or written to an out
-// bank) and the three fields of the other phase.  Shapes are derived from the
-// material grid (nz, ny, nx) by the complete-Yee rule and validated on the host.
-// Timed source slabs folded into a 2D (TMxy) phase launch, float32 fields:
-// each updated cell adds its slabs' terms in declaration order, as the
-// source launches after the phase would (execute.py:374-461; the kernel may
-// fuse a term's multiply and add, so the sums agree to rounding), skipping
-// the PEC-constrained ends.  comp: the target within the phase (0 Hx, 1 Hy
-// for H; 2 Ez for E).
+// Timed source slabs of one target, folded into a phase launch, float32 fields:
+// each updated cell adds its slabs' terms, as the source launches after the
+// phase would (execute.py:374-461), skipping the PEC-constrained ends.  2D adds
+// term after term in declaration order, 3D the terms' sum; both may fuse a
+// term's multiply and add, so they agree with the launches to rounding.
 struct PhaseSrc {
   const float* coeff;      // [n, sz, sy, sx]
   const float* wave;       // [n, T]
@@ -115,6 +111,9 @@ struct PhaseSrc {
   int32_t mlo[3], mhi[3];  // PEC-constrained ends (z, y, x)
 };
 
+// Fields of one phase: three targets (updated in place, or written to an out
+// bank) and the three fields of the other phase.  Shapes are derived from the
+// material grid (nz, ny, nx) by the complete-Yee rule and validated on the host.
 struct PhaseParams {
   const void* tin[3];   // targets read
   void* tout[3];        // targets written (== tin for in-place launches)
@@ -420,7 +419,7 @@ void launch_dft_capture(hipStream_t s, const DftCapParams& p);
 
 // Several TMxy steps in one launch (tm_steps.hip): float32 fields and CPML
 // memories, scalar H coefficients, one CPML thickness L on every edge (0:
-// none), isotropic metrics.  Bank A (``_in``) is read, bank B written.
+// none), isotropic metrics.  One bank is read, the other written.
 constexpr int kTmMaxSteps = 8;
 constexpr int kTmRows = 32;   // rows of a tile (64 columns)
 constexpr int kMaxTmSlabs = 12;

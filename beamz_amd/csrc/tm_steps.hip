@@ -591,9 +591,9 @@ __global__ void __launch_bounds__(64 * NW) tm_steps(TmParams) {
 }
 
 // Batched simulations: one block per tile of any member, the members'
-// descriptors in device memory.  (One wave per 62-column item, one step per
-// launch and bank B written every step: 121 GCUPS on 64 simulations of 26 M
-// cells; this kernel: see launch_tm_batch.)
+// descriptors in device memory.  64 simulations of 26 M cells: 424 GCUPS; one
+// wave per 62-column item with one step per launch reached 121.  Members
+// without CPML run the CPML form too, whose curl rounds both terms.
 template <int NW, int RPT>
 __global__ void __launch_bounds__(64 * NW) tm_batch(TmBatchParams p) {
   __shared__ float rows[2][NW][2][64];
