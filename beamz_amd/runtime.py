@@ -172,14 +172,21 @@ class Workspace2D(tuple):
         return torch.Size, ((),)  # an empty tuple that ``weights_only`` loading accepts
 
 
-def with_workspace_2d(state, prog):
+def _stream(prog):
+    """The current stream's handle, read once per call (None: no GPU)."""
+    return native.current_stream_handle() if prog.device.type == "cuda" else None
+
+
+def with_workspace_2d(state, prog, handle=None):
     """The state with the 2D program's multi-step workspace in its second-bank
     slot (:class:`Workspace2D`), allocated where the state has none of its own
-    for the current stream."""
+    for the current stream (``handle``, from :func:`_stream`)."""
     n = prog.workspace_floats
     if n == 0 or prog.is_3d:
         return state
-    stream = torch.cuda.current_stream().cuda_stream if prog.device.type == "cuda" else 0
+    if handle is None:
+        handle = _stream(prog)
+    stream = (handle.value or 0) if handle is not None else 0
     held = state.fields_b
     if isinstance(held, Workspace2D) and held.fits(state.ez, stream, n):
         return state
@@ -197,9 +204,10 @@ def run_steps(state, prog, nsteps):
     if uses_two_banks(prog):
         return run_source_group_steps(state, prog, nsteps)
     layout = abi.PROGRAM_LAYOUT_CPML_IN_PLACE if prog.cpml_enabled else abi.PROGRAM_LAYOUT_YEE_IN_PLACE
-    state = with_workspace_2d(state, prog)
+    stream = _stream(prog)
+    state = with_workspace_2d(state, prog, stream)
     native.call_program((*_graph_io(prog, state), *_workspace_args(state, prog)),
-                        _program_attrs(prog, nsteps, layout))
+                        _program_attrs(prog, nsteps, layout), stream)
     return state
 
 
@@ -212,11 +220,12 @@ def run_source_group_steps(state, prog, nsteps, *, noalloc=False):
         native.call_program(args, _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_SOURCE_TEMPORAL_CPML),
                             noalloc=noalloc)
         return _swap_banks(state, nsteps)
-    state = state if noalloc else with_workspace_2d(state, prog)
+    stream = _stream(prog)
+    state = state if noalloc else with_workspace_2d(state, prog, stream)
     args = (*_graph_io(prog, state), *_source_group_arguments(prog), state.current_step,
             *_workspace_args(state, prog))
     native.call_program(args, _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_SOURCE_IN_PLACE),
-                        noalloc=noalloc)
+                        stream, noalloc=noalloc)
     return state
 
 
@@ -243,10 +252,11 @@ def run_program_steps(state, prog, nsteps, *, noalloc=False):
                             _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_MONITOR_TEMPORAL_CPML,
                                            monitor_count=len(prog.monitors)), noalloc=noalloc)
         return _swap_banks(state, nsteps)
-    state = state if noalloc else with_workspace_2d(state, prog)
+    stream = _stream(prog)
+    state = state if noalloc else with_workspace_2d(state, prog, stream)
     native.call_program((*_graph_io(prog, state), *tail, *_workspace_args(state, prog)),
                         _program_attrs(prog, nsteps, abi.PROGRAM_LAYOUT_MONITOR_IN_PLACE,
-                                       monitor_count=len(prog.monitors)), noalloc=noalloc)
+                                       monitor_count=len(prog.monitors)), stream, noalloc=noalloc)
     return state
 
 
