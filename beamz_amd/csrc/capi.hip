@@ -2618,7 +2618,7 @@ int32_t bzh_adjoint2d_recompute(void* stream, const bzh_buffer* args, int32_t na
     BZH_REQUIRE(!temporal && in.bank_a[kEz]->rank == 2, "the recompute steps a 2D in-place program");
     int64_t slots = 0;
     Adjoint2dParams p = describe_adjoint(*adj, &slots);
-    BZH_REQUIRE(in.nsteps >= 1 && slot >= 0 && slot + in.nsteps <= slots, "record slots out of range");
+    BZH_REQUIRE(in.nsteps >= 1 && slot >= 0 && int64_t{slot} + in.nsteps <= slots, "record slots out of range");
     const Grid g = infer_grid(in.bank_a);
     BZH_REQUIRE(g.dtype == BZH_F32 && g.ny == p.ny && g.nx == p.nx,
                 "the recomputed program does not match the adjoint grid");
