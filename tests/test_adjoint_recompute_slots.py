@@ -4,6 +4,8 @@ are refused before anything is launched.)"""
 
 from __future__ import annotations
 
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 import torch
@@ -34,5 +36,6 @@ def test_record_slots_out_of_range(slot, nsteps):
     for q, v in enumerate((5, 9, 6, 11)):
         adj.design[q] = v
     call = runtime.prepare_chunk(state, prog, 1)
-    with pytest.raises(native.HipLaunchError, match="record slots out of range"):
-        call.recompute(adj, nsteps, slot, stream=0)
+    # (on a thread of its own: the library keeps the last error per thread)
+    with ThreadPoolExecutor(1) as pool, pytest.raises(native.HipLaunchError, match="record slots out of range"):
+        pool.submit(call.recompute, adj, nsteps, slot, 0).result()
